@@ -18,10 +18,12 @@
 //                                    SwiGLU epilogue -> h.Ud -> XUd.Vd; stages
 //                                    with too few output tiles split K into
 //                                    fp32 slices summed in split order
-//   anything else (fp32, Linear-layout or transposed operands, odd sizes):
-//                                    the general 128x128 GEMM (gemm.hpp) and
-//                                    the per-stage decode kernels (decode.hpp),
-//                                    whose split-K sums use fp32 atomics
+//   1-64 tokens, Linear-layout or fp8 factors, dimensions off the decode
+//   layer's tiles (multiples of 8), and the gate/up and x.u.v entry points:
+//                                    one streaming launch per stage (stream.hpp)
+//   anything else (fp32, odd sizes):
+//                                    the general 128x128 GEMM (gemm.hpp), whose
+//                                    split-K sums use fp32 atomics
 // Every buffer, including the workspace that holds the rank-r intermediates,
 // h and the split-K slices, is owned by the caller.
 #include <stdarg.h>
@@ -41,6 +43,7 @@
 #include "decode_layer.hpp"
 #include "gemm_big.hpp"
 #include "gemm_f8f8.hpp"
+#include "stream.hpp"
 #include "svdmlp.h"
 
 using namespace svdmlp;
@@ -192,6 +195,7 @@ struct Ws {
   size_t need;     // bytes every call needs (the regions above)
   size_t cslices;  // partial XU_d tiles of the contracted decode layer (T <= kDlContractMaxT), last: a
                    // workspace without them runs the other decode layers
+  size_t xslices;  // slices of the streaming stages at up to 32 tokens, last: without them they use `slices`
   size_t total;
 };
 
@@ -289,6 +293,11 @@ Ws ws_layout(int64_t T, int64_t d, int64_t ff, int64_t r) {
   off += (T <= kDlContractMaxT && ff % 64 == 0 && ff / 64 + r / 128 <= kDlMaxGrid)
              ? a256(dl_contract_bytes(r / 128, ff / 64, T))
              : 0;
+  // the streaming stages' slices where `slices` is short of them: 256 units
+  // of two branches and 256 columns, T rows each (kDecodeMaxT tokens with 128
+  // columns fit `slices`)
+  w.xslices = off;
+  off += T <= 32 ? a256(T * 1024 * 128 * 4) : 0;
   w.total = off;
   return w;
 }
@@ -1302,43 +1311,82 @@ int big_v(const Common& c, const uint16_t* xu, const void* v, bool v_lin, int T,
 // Decode stages
 // ---------------------------------------------------------------------------
 
-int decode_mt(int64_t T) { return T <= 16 ? 1 : (T <= 32 ? 2 : 4); }
+// One streaming stage (stream.hpp) of up to two segments: bf16 out_i =
+// A_i . W_i side by side, or (dual) out_0 = SiLU(A_0 . W_0) * (A_1 . W_1).
+struct StreamOut {
+  uint16_t* p;
+  int64_t ld;
+  bool t = false;                   // written transposed, (N, T)
+  const uint16_t* resid = nullptr;  // the MLP block's residual
+};
 
-int decode_stage(const Common& c, int stage, int T, int K, int nseg, const Operand* a, int srca,
-                 const void* const* w, const float* const* sw, bool w_lin, const int* N, float* const* out,
-                 const char* what) {
-  DecodeParams p{};
-  p.nseg = nseg;
-  p.T = T;
-  p.K = K;
-  int tiles = 0;
-  for (int s = 0; s < nseg; ++s) {
-    p.a[s] = a[s];
-    p.seg[s].w = w[s];
-    p.seg[s].scale = sw ? sw[s] : nullptr;
-    p.seg[s].out = out[s];
-    p.seg[s].ldw = w_lin ? K : N[s];
-    p.seg[s].ldo = N[s];
-    p.seg[s].N = N[s];
-    p.seg[s].ntiles = (N[s] + kDecTileN - 1) / kDecTileN;
-    tiles += p.seg[s].ntiles;
-  }
-  // K slice per block: enough blocks to cover the chip ~2x, slices of >= 128.
-  int64_t ks = ((int64_t)K * tiles + 511) / 512;
-  ks = std::max<int64_t>(128, (ks + 127) / 128 * 128);
-  ks = std::min<int64_t>(ks, ((int64_t)K + 31) / 32 * 32);
-  p.k_split = (int)ks;
-  const int splits = (int)(((int64_t)K + ks - 1) / ks);
-  DecodeDesc d{decode_mt(T), srca, srcb_of(c.wt), w_lin};
-  const char* why = nullptr;
-  StageScope ss(stage, c.st);
-  return check(launch_decode(d, p, tiles * splits, c.st, &why), what, why);
+// K splits of a streaming stage with `tiles` column tiles, each unit of which
+// stores `slice` bytes: as many units as CUs (one 8-wave block keeps 128 KB
+// in flight), each of at least 256 k, so that all of them stream together and
+// end together, and as far as their slices fit the workspace's area.  Two
+// units a CU only double the slices and their sums: 8B Linear layer at 16
+// tokens 91.4 us with 256 units, 98.1 with 512; 70B fp8 layer at 4 tokens
+// 129.7 and 140.1; 8B x.u.v at 32 tokens 32.8 and 42.2.
+constexpr int64_t kStreamUnits = 256;
+
+int stream_splits(int64_t K, int64_t tiles, int64_t slice, int64_t area, int* ks) {
+  int64_t s = std::min(std::min(kStreamUnits / tiles, K / 256), area / (tiles * slice));
+  if (tiles > kDlMaxTiles) s = 1;
+  s = std::max<int64_t>(s, 1);
+  *ks = (int)(((K + s - 1) / s + 63) / 64 * 64);
+  return (int)((K + *ks - 1) / *ks);
 }
 
+int64_t stream_area(const Ws& L, size_t ws_bytes, size_t* off) {
+  const bool x = ws_bytes >= L.total && L.total > L.xslices;  // the larger area at the end
+  *off = x ? L.xslices : L.slices;
+  return std::min<int64_t>((int64_t)(x ? L.total - L.xslices : L.need - L.slices), 0x7ffffff0);
+}
+
+int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, bool dual, const uint16_t* const* a,
+                 const void* const* w, const float* const* sw, bool w_lin, const int64_t* N, const StreamOut* out,
+                 char* ws, const Ws& L, size_t ws_bytes, const char* what) {
+  StreamParams p{};
+  const int wk = w_lin ? SW_LINEAR : (c.wt == SVDMLP_FP8_E4M3 ? SW_FP8 : SW_NATURAL);
+  // fp8 rows in 256-byte pieces (16 columns a lane) where the registers and
+  // the row length allow it: 70B layer at 4 tokens 130 us, 140 in 128-byte pieces
+  const int cg = wk == SW_FP8 && T <= 32 && N[0] % 16 == 0 && N[nseg - 1] % 16 == 0 ? 2 : 1;
+  const int64_t bn = kStTileN * cg;
+  int ks = 0;
+  p.T = (int)T;
+  for (int i = 0; i < nseg; ++i) p.tiles += !dual || i == 0 ? (int)((N[i] + bn - 1) / bn) : 0;
+  size_t off = 0;
+  const int64_t area = stream_area(L, ws_bytes, &off);
+  p.slices = reinterpret_cast<float*>(ws + off);
+  p.slice_bytes = (uint32_t)area;
+  p.splits = stream_splits(K, p.tiles, (dual ? 2 : 1) * T * bn * 4, area, &ks);
+  p.exchange = p.splits > 1 || out[0].t;
+  p.out_t = out[0].t;
+  p.sync = reinterpret_cast<uint64_t*>(ws + L.sync);
+  p.resid = out[0].resid;
+  for (int i = 0; i < nseg; ++i)
+    p.seg[i] = StreamSeg{a[i], w[i], sw ? sw[i] : nullptr, out[dual ? 0 : i].p, w_lin ? K : N[i], out[dual ? 0 : i].ld,
+                         (int)K, (int)N[i], (int)((N[i] + bn - 1) / bn), ks};
+  const char* why = nullptr;
+  StageScope ss(stage, c.st);
+  return check(launch_stream(p, wk, cg, dual, c.st, &why), what, why);
+}
+
+// A streaming stage can write its tiles transposed: each then goes through
+// the slice area whole.
+bool stream_out_t_ok(int64_t T, int64_t N, const Ws& L, size_t ws_bytes) {
+  const int64_t tiles = (N + 2 * kStTileN - 1) / (2 * kStTileN) * 2;
+  size_t off = 0;
+  return tiles <= kDlMaxTiles && tiles * 2 * T * kStTileN * 4 <= stream_area(L, ws_bytes, &off);
+}
+
+// Streaming stages take bf16 activations and any bf16 or fp8 factors in rows
+// of whole 16-byte pieces (fp8: 8), with the 32-bit offsets of one step and of
+// the activations in range.
 bool decode_ok(const Common& c, int64_t T, std::initializer_list<int64_t> dims, bool vec) {
   if (c.f32 || T > kDecodeMaxT || !vec) return false;
   for (int64_t v : dims)
-    if (v % 8) return false;
+    if (v % 8 || v >= (int64_t)1 << 22 || T * v * 2 >= ((int64_t)1 << 31)) return false;
   return true;
 }
 
@@ -1385,7 +1433,7 @@ int dl_plan(int64_t K, int64_t tiles, int grid, int* units, int max_s = 0) {
 // T <= kDlContractMaxT with a block for every h strip and XU_d tile.
 bool decode_contract_ok(int64_t T, int64_t ff, int64_t r_gu, int64_t r_d, const Ws& L, size_t ws_bytes) {
   // the gate/up run-out prefetches the down half's first 5 ring stages of 64 k
-  if (T > kDlContractMaxT || L.total == L.cslices || ws_bytes < L.total || r_gu < 320) return false;
+  if (T > kDlContractMaxT || L.xslices == L.cslices || ws_bytes < L.xslices || r_gu < 320) return false;
   const int grid = decode_layer_contract_grid();
   return grid > 0 && ff / 64 + r_d / 128 <= grid;
 }
@@ -1817,32 +1865,29 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
   char* ws = static_cast<char*>(workspace);
 
   if (decode_ok(c, T, {d, ff, r}, vec)) {
-    float* xu32 = reinterpret_cast<float*>(ws + L.xu32);
-    float* g32 = reinterpret_cast<float*>(ws + L.gu32);
-    float* u32 = g32 + T * ff;
+    uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
+    const uint16_t* x16 = static_cast<const uint16_t*>(x);
     {
-      StageScope z(ST_ZERO, c.st);
-      rc = check(launch_fill_zero(xu32, (int64_t)(L.h - L.xu32) / 4, c.st), "zero accumulators");
+      const uint16_t* a[2] = {x16, x16};
+      const void* w[2] = {ug, uu};
+      const float* s[2] = {s_ug, s_uu};
+      const int64_t n[2] = {r, r};
+      const StreamOut o[2] = {{xu, r}, {xu + T * r, r}};
+      if ((rc = stream_stage(c, ST_DEC_GU_XU, T, d, 2, false, a, w, fp8 ? s : nullptr, u_lin, n, o, ws, L, ws_bytes, "decode X.U")))
+        return rc;
     }
-    if (rc) return rc;
-    const Operand ax{x, nullptr, d};
-    const Operand a1[2] = {ax, ax};
-    const void* w1[2] = {ug, uu};
-    const float* s1[2] = {s_ug, s_uu};
-    const int n1[2] = {(int)r, (int)r};
-    float* o1[2] = {xu32, xu32 + T * r};
-    rc = decode_stage(c, ST_DEC_GU_XU, T, d, 2, a1, SRC_BF16, w1, fp8 ? s1 : nullptr, u_lin, n1, o1, "decode X.U");
-    if (rc) return rc;
-    const Operand a2[2] = {Operand{xu32, nullptr, r}, Operand{xu32 + T * r, nullptr, r}};
-    const void* w2[2] = {vg, vu};
-    const float* s2[2] = {s_vg, s_vu};
-    const int n2[2] = {(int)ff, (int)ff};
-    float* o2[2] = {g32, u32};
-    rc = decode_stage(c, ST_DEC_GU_XUV, T, r, 2, a2, SRC_F32, w2, fp8 ? s2 : nullptr, v_lin, n2, o2, "decode XU.V");
-    if (rc) return rc;
+    const uint16_t* a[2] = {xu, xu + T * r};
+    const void* w[2] = {vg, vu};
+    const float* s[2] = {s_vg, s_vu};
+    const int64_t n[2] = {ff, ff};
+    const bool direct_t = out_t && stream_out_t_ok(T, ff, L, ws_bytes);
+    uint16_t* hn = out_t && !direct_t ? reinterpret_cast<uint16_t*>(ws + L.h) : static_cast<uint16_t*>(h);
+    const StreamOut o[1] = {{hn, direct_t ? T : ff, direct_t}};
+    if ((rc = stream_stage(c, ST_DEC_GU_XUV, T, r, 2, true, a, w, fp8 ? s : nullptr, v_lin, n, o, ws, L, ws_bytes, "decode XU.V")) ||
+        !out_t || direct_t)
+      return rc;
     StageScope fin(ST_FINALIZE, c.st);
-    return check(launch_finalize(g32, u32, ff, static_cast<uint16_t*>(h), out_t ? T : ff, T, ff, true, out_t, c.st),
-                 "SwiGLU finalize");
+    return check(launch_transpose_bf16(hn, ff, static_cast<uint16_t*>(h), T, (int)T, (int)ff, c.st), "h transpose");
   }
 
   if (big_ok(c, vec, {T * d * 2, d * r * 2, r * ff * 2, T * ff * 2}, {d, r})) {
@@ -1912,31 +1957,15 @@ int svdmlp_xuv(const void* x, const void* u, const void* v, const float* s_u, co
   }
 
   if (!x_t && decode_ok(c, T, {din, dout, r}, vec)) {
-    float* xd32 = reinterpret_cast<float*>(ws + L.xu32) + 2 * T * r;
-    float* y32 = reinterpret_cast<float*>(ws + L.y32);
-    {
-      StageScope z(ST_ZERO, c.st);
-      rc = check(launch_fill_zero(xd32, T * r, c.st), "zero accumulators");
-      if (!rc) rc = check(launch_fill_zero(y32, T * dout, c.st), "zero accumulators");
-    }
-    if (rc) return rc;
-    const Operand a1[1] = {Operand{x, nullptr, din}};
-    const void* w1[1] = {u};
-    const float* s1[1] = {s_u};
-    const int n1[1] = {(int)r};
-    float* o1[1] = {xd32};
-    rc = decode_stage(c, ST_DEC_D_XU, T, din, 1, a1, SRC_BF16, w1, fp8 ? s1 : nullptr, u_lin, n1, o1, "decode X.U");
-    if (rc) return rc;
-    const Operand a2[1] = {Operand{xd32, nullptr, r}};
-    const void* w2[1] = {v};
-    const float* s2[1] = {s_v};
-    const int n2[1] = {(int)dout};
-    float* o2[1] = {y32};
-    rc = decode_stage(c, ST_DEC_D_XUV, T, r, 1, a2, SRC_F32, w2, fp8 ? s2 : nullptr, v_lin, n2, o2, "decode XU.V");
-    if (rc) return rc;
-    StageScope fin(ST_FINALIZE, c.st);
-    return check(launch_finalize(y32, nullptr, dout, static_cast<uint16_t*>(y), dout, T, dout, false, false, c.st),
-                 "output finalize");
+    uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
+    const uint16_t* a1 = static_cast<const uint16_t*>(x);
+    const StreamOut o1{xu, r}, o2{static_cast<uint16_t*>(y), dout};
+    if ((rc = stream_stage(c, ST_DEC_D_XU, T, din, 1, false, &a1, &u, fp8 ? &s_u : nullptr, u_lin, &r, &o1, ws, L, ws_bytes,
+                           "decode X.U")))
+      return rc;
+    const uint16_t* a2 = xu;
+    return stream_stage(c, ST_DEC_D_XUV, T, r, 1, false, &a2, &v, fp8 ? &s_v : nullptr, v_lin, &dout, &o2, ws, L, ws_bytes,
+                        "decode XU.V");
   }
 
   if (!x_t && big_ok(c, vec, {T * din * 2, din * r * 2, r * dout * 2, T * dout * 2}, {din, r})) {
@@ -2132,54 +2161,34 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
   if ((rc = normed())) return rc;
 
   if (decode_ok(c, T, {d, ff, r_gu, r_d}, vec)) {
-    float* xu32 = reinterpret_cast<float*>(ws + L.xu32);
-    float* xg = xu32;
-    float* xuu = xu32 + T * r;
-    float* xd = xu32 + 2 * T * r;
-    float* g32 = reinterpret_cast<float*>(ws + L.gu32);
-    float* u32 = g32 + T * ff;
-    float* y32 = reinterpret_cast<float*>(ws + L.y32);
+    uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
+    uint16_t* hb = reinterpret_cast<uint16_t*>(ws + L.h);
+    const uint16_t* x16 = static_cast<const uint16_t*>(x);
     {
-      StageScope z(ST_ZERO, c.st);
-      rc = check(launch_fill_zero(xu32, (int64_t)(L.part - L.xu32) / 4, c.st), "zero accumulators");
-    }
-    if (rc) return rc;
-    const Operand ax{x, nullptr, d};
-    {
-      const Operand a[2] = {ax, ax};
+      const uint16_t* a[2] = {x16, x16};
       const void* w[2] = {ug, uu};
       const float* s[2] = {S[0], S[2]};
-      const int n[2] = {(int)r_gu, (int)r_gu};
-      float* o[2] = {xg, xuu};
-      if ((rc = decode_stage(c, ST_DEC_GU_XU, T, d, 2, a, SRC_BF16, w, s, u_lin, n, o, "decode X.U"))) return rc;
+      const int64_t n[2] = {r_gu, r_gu};
+      const StreamOut o[2] = {{xu, r_gu}, {xu + T * r_gu, r_gu}};
+      if ((rc = stream_stage(c, ST_DEC_GU_XU, T, d, 2, false, a, w, s, u_lin, n, o, ws, L, ws_bytes, "decode X.U"))) return rc;
     }
     {
-      const Operand a[2] = {Operand{xg, nullptr, r_gu}, Operand{xuu, nullptr, r_gu}};
+      const uint16_t* a[2] = {xu, xu + T * r_gu};
       const void* w[2] = {vg, vu};
       const float* s[2] = {S[1], S[3]};
-      const int n[2] = {(int)ff, (int)ff};
-      float* o[2] = {g32, u32};
-      if ((rc = decode_stage(c, ST_DEC_GU_XUV, T, r_gu, 2, a, SRC_F32, w, s, v_lin, n, o, "decode XU.V"))) return rc;
+      const int64_t n[2] = {ff, ff};
+      const StreamOut o{hb, ff};
+      if ((rc = stream_stage(c, ST_DEC_GU_XUV, T, r_gu, 2, true, a, w, s, v_lin, n, &o, ws, L, ws_bytes, "decode XU.V"))) return rc;
     }
-    {
-      const Operand a[1] = {Operand{g32, u32, ff}};
-      const void* w[1] = {ud};
-      const float* s[1] = {S[4]};
-      const int n[1] = {(int)r_d};
-      float* o[1] = {xd};
-      if ((rc = decode_stage(c, ST_DEC_D_XU, T, ff, 1, a, SRC_SWIGLU, w, s, u_lin, n, o, "decode h.Ud"))) return rc;
-    }
-    {
-      const Operand a[1] = {Operand{xd, nullptr, r_d}};
-      const void* w[1] = {vd};
-      const float* s[1] = {S[5]};
-      const int n[1] = {(int)d};
-      float* o[1] = {y32};
-      if ((rc = decode_stage(c, ST_DEC_D_XUV, T, r_d, 1, a, SRC_F32, w, s, v_lin, n, o, "decode XUd.Vd"))) return rc;
-    }
-    StageScope fin(ST_FINALIZE, c.st);
-    return check(launch_finalize(y32, nullptr, d, static_cast<uint16_t*>(y), d, T, d, false, false, c.st),
-                 "output finalize");
+    const StreamOut o1{xu, r_d};
+    const uint16_t* a1 = hb;
+    if ((rc = stream_stage(c, ST_DEC_D_XU, T, ff, 1, false, &a1, &ud, &S[4], u_lin, &r_d, &o1, ws, L, ws_bytes, "decode h.Ud")))
+      return rc;
+    // the MLP block's residual add rides on the last stage's output
+    const StreamOut o2{static_cast<uint16_t*>(y), d, false, blk ? static_cast<const uint16_t*>(blk->x) : nullptr};
+    if (blk) blk->resid_done = true;
+    const uint16_t* a2 = xu;
+    return stream_stage(c, ST_DEC_D_XUV, T, r_d, 1, false, &a2, &vd, &S[5], v_lin, &d, &o2, ws, L, ws_bytes, "decode XUd.Vd");
   }
 
   // Prefill: h stays in the workspace between the two halves.

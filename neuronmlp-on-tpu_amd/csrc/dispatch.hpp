@@ -5,7 +5,9 @@
 
 #include <atomic>
 
-#include "decode.hpp"
+#include <algorithm>
+
+#include "gemm.hpp"
 
 namespace svdmlp {
 
@@ -20,13 +22,6 @@ struct GemmDesc {
   bool out_t;    // transposed output
   bool out_f32;  // fp32 output (EPI_STORE / EPI_SWIGLU)
   bool vec;      // 16-byte vector path (aligned, multiples of 8)
-};
-
-struct DecodeDesc {
-  int mt;        // 16-row token tiles: 1, 2 or 4
-  int srca;      // SRC_BF16, SRC_F32 or SRC_SWIGLU
-  int srcb;      // SRC_BF16 or SRC_FP8
-  bool b_kc;     // Linear-layout weights
 };
 
 struct BigDesc {
@@ -54,8 +49,10 @@ hipError_t launch_gemm_f32(const GemmDesc& d, const GemmParams& p, int splits, i
                            const char** why);
 hipError_t launch_big(const BigDesc& d, const BigParams& p, int splits, int batch, hipStream_t st,
                       const char** why);
-hipError_t launch_decode(const DecodeDesc& d, const DecodeParams& p, int blocks, hipStream_t st,
-                         const char** why);
+// Decode-shape streaming stage (stream.hpp): wk a StreamW, tiles of 128 cg
+// columns (cg 2: fp8 up to 32 tokens), dual the gate/up pair of a column tile.
+struct StreamParams;
+hipError_t launch_stream(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st, const char** why);
 hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t st);
 // MLP block prologue / epilogue: y = act(gain * rmsnorm(x)), y = act(x + y).
 hipError_t launch_rmsnorm(const void* x, const float* gain, void* y, int64_t T, int64_t d, float eps, bool bf16,
@@ -109,8 +106,6 @@ hipError_t launch_f8_gemm(const F8Params& p, int splits, int nw, hipStream_t st,
 // (m%16)*128 + k%128; n a multiple of 128, ldq unused), the fp8 GEMM's a_blk.
 hipError_t launch_quant_rows_e4m3(const uint16_t* h, int64_t ldh, uint8_t* q, int64_t ldq, float* s, int rows, int n,
                                   hipStream_t st, const char** why, bool blk = false);
-hipError_t launch_finalize(const float* g, const float* u, int64_t ldi, uint16_t* out, int64_t ldo, int rows,
-                           int cols, bool swiglu, bool out_t, hipStream_t st);
 
 // A per-device constant (a persistent kernel's grid size) computed once per
 // device and slot: the lookups behind it (device attributes, occupancy) cost

@@ -1,0 +1,125 @@
+"""The streaming stages of decode shapes (csrc/stream.hpp): Linear-layout and
+fp8 factors, dimensions off the decode layer's tiles, and the gate/up and
+x.u.v entry points, at the edges of their tiles.
+
+Tolerance: bf16 results round the rank intermediate, h and y once each, a
+relative error of at most 2^-9 per value and rounding (rms 1.1e-3); through
+the layer's products and SiLU(g) * u the three add up to 3e-3 to 6e-3 of the
+result's norm, so 1e-2.  fp8 factors are widened exactly and are compared
+with the same math on the dequantised factors.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from svdmlp import _lib, fp8, inputs, ops
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-2
+
+
+def _np(t):
+    return t.float().cpu().numpy()
+
+
+def _rel(got, want):
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
+def _layer(shape, T, seed, kind, dev):
+    """(x, factors) as the operators take them and as float32 arrays."""
+    x, f = inputs.make_layer(shape, T=T, seed=seed)
+    xb = inputs.as_float32(x, torch.bfloat16)
+    xt = inputs.to_torch(xb, torch.bfloat16, dev)
+    if kind == "fp8":
+        q = [fp8.quantize_per_channel(torch.from_numpy(a)) for a in f]
+        wide = [O.e4m3_decode(a.data.view(torch.uint8).numpy()) * a.scale.numpy() for a in q]
+        return xb, wide, xt, [ops.QuantizedFactor(a.data.to(dev), a.scale.to(dev)) for a in q]
+    wide = [inputs.as_float32(a, torch.bfloat16) for a in f]
+    ft = [inputs.to_torch(a, torch.bfloat16, dev) for a in wide]
+    if kind == "linear":
+        ft = [a.t().contiguous().t() for a in ft]
+    return xb, wide, xt, ft
+
+
+# 16-row token tiles full, one over and short of full; ranks and widths off the
+# 128-column (fp8: 256) tiles, off the 64-k blocks and 32-k steps and down to
+# one 8-wide piece; more K splits than one batch of slices (d = 4160: 16)
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("kind", ["natural", "linear", "fp8"])
+@pytest.mark.parametrize("shape", [inputs.LayerShape(136, 200, 72, 40), inputs.LayerShape(4160, 528, 136, 264),
+                                   inputs.LayerShape(264, 2064, 400, 272)])
+def test_stream_entry_points(gpu, shape, kind, T):
+    xb, wide, xt, ft = _layer(shape, T, 300 + T, kind, gpu)
+    h = ops.fused_gate_up(xt, *ft[:4])
+    assert _rel(_np(h), O.fused_gate_up_ref(xb, *wide[:4], dtype="bfloat16")) < TOL
+    y = ops.fused_xuv(h, *ft[4:])
+    assert _rel(_np(y), O.fused_xuv_ref(_np(h), *wide[4:], dtype="bfloat16")) < TOL
+    out = ops.svd_mlp(xt, *ft)
+    assert _rel(_np(out), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+    # split-K slices are summed in split order whichever unit is last: the same bits on replay
+    for _ in range(3):
+        assert torch.equal(ops.fused_gate_up(xt, *ft[:4]).view(torch.int16), h.view(torch.int16))
+        assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
+    if T % 8 == 0:  # transposed operands: the natural result's bits
+        hT = ops.fused_gate_up(xt, *ft[:4], out_transposed=True)
+        assert torch.equal(hT.view(torch.int16), h.t().contiguous().view(torch.int16))
+        yT = ops.fused_xuv(h.t().contiguous(), *ft[4:], x_transposed=True)
+        assert torch.equal(yT.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("kind", ["linear", "fp8"])
+def test_stream_block(gpu, kind):
+    """The MLP block: RMSNorm ahead, the residual added by the last stage."""
+    shape = inputs.LayerShape(1024, 2048, 512, 384)
+    xb, wide, xt, ft = _layer(shape, 24, 11, kind, gpu)
+    gain = torch.rand(shape.d, device=gpu) + 0.5
+    y = ops.svd_mlp_block(xt, gain, *ft)
+    mlp = ops.svd_mlp((xt.float() * torch.rsqrt(xt.float().pow(2).mean(1, keepdim=True) + 1e-5) * gain).bfloat16(), *ft)
+    # bf16(x + bf16(mlp)); the RMSNorm's own rounding may differ by one bf16 step
+    assert _rel(_np(y), _np((xt.float() + mlp.float()).bfloat16())) < TOL
+
+
+def test_stream_small_workspace(gpu):
+    """A workspace without the larger slice area at its end (fewer K splits)."""
+    shape = inputs.LayerShape(1024, 2048, 512)
+    xb, wide, xt, ft = _layer(shape, 16, 12, "linear", gpu)
+    ws = ops.svd_mlp_workspace(xt, r=shape.r, ff=shape.ff)
+    extra = 16 * 1024 * 128 * 4
+    short = torch.zeros(ws.numel() - extra, dtype=torch.uint8, device=gpu)
+    want = O.svd_mlp_ref(xb, *wide, dtype="bfloat16")
+    for w in (ws, short):
+        assert _rel(_np(ops.svd_mlp(xt, *ft, workspace=w)), want) < TOL
+
+
+def test_stream_after_a_timeout(gpu):
+    """A workspace whose timeout flag is set gives NaN until it is reset (the
+    tile counters may hold anything then)."""
+    shape = inputs.LayerShape(1024, 2048, 512)
+    xb, wide, xt, ft = _layer(shape, 8, 13, "linear", gpu)
+    ws = ops.svd_mlp_workspace(xt, r=shape.r, ff=shape.ff)
+    ws[2304:2312].view(torch.int64).fill_(1)
+    assert torch.isnan(ops.svd_mlp(xt, *ft, workspace=ws)).all()
+    assert ops.workspace_status(ws, reset=True) is True
+    assert _rel(_np(ops.svd_mlp(xt, *ft, workspace=ws)), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+
+
+def test_stream_two_streams(gpu):
+    """Two streams at once, a workspace each: no unit waits for another."""
+    shape = inputs.LayerShape(2048, 4096, 512)
+    sets = [_layer(shape, T, 20 + T, kind, gpu) for T, kind in ((16, "fp8"), (40, "linear"))]
+    ws = [ops.svd_mlp_workspace(s[2], r=shape.r, ff=shape.ff, w_code=_lib.SVDMLP_BF16) for s in sets]
+    want = [ops.svd_mlp(s[2], *s[3], workspace=w).clone() for s, w in zip(sets, ws)]
+    streams = [torch.cuda.Stream() for _ in sets]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(20):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(ops.svd_mlp(sets[i][2], *sets[i][3], workspace=ws[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(g.view(torch.int16), want[i].view(torch.int16)) for g in got[i])
