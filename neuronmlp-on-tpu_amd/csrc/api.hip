@@ -21,8 +21,9 @@
 //   1-64 tokens, Linear-layout or fp8 factors, dimensions off the decode
 //   layer's tiles (multiples of 8), and the gate/up and x.u.v entry points:
 //                                    one streaming launch per stage (stream.hpp)
-//   anything else (fp32, odd sizes):
-//                                    the general 128x128 GEMM (gemm.hpp), whose
+//   fp32, aligned:                   one fp32 streaming launch per stage
+//                                    (stream_f32.hpp)
+//   anything else (odd sizes):       the general 128x128 GEMM (gemm.hpp), whose
 //                                    split-K sums use fp32 atomics
 // Every buffer, including the workspace that holds the rank-r intermediates,
 // h and the split-K slices, is owned by the caller.
@@ -44,6 +45,7 @@
 #include "gemm_big.hpp"
 #include "gemm_f8f8.hpp"
 #include "stream.hpp"
+#include "stream_f32.hpp"
 #include "svdmlp.h"
 
 using namespace svdmlp;
@@ -355,7 +357,7 @@ int prefill_xu(const Common& c, const Operand& a, bool a_kc, const void* const* 
   GemmParams p{};
   for (int b = 0; b < batch; ++b) {
     p.a[b] = a;
-    p.b[b] = Operand{u[b], nullptr, u_lin ? K : r};
+    p.b[b] = Operand{u[b], u_lin ? K : r};
     p.scale[b] = su ? su[b] : nullptr;
   }
   p.M = T;
@@ -399,10 +401,10 @@ int prefill_swiglu(const Common& c, int a_src, const void* xu, int64_t xu_bstrid
                    void* out) {
   GemmParams p{};
   const size_t esz = (a_src == SRC_F32) ? 4 : 2;
-  p.a[0] = Operand{xu, nullptr, r};
-  p.a[1] = Operand{static_cast<const char*>(xu) + xu_bstride * esz, nullptr, r};
-  p.b[0] = Operand{vg, nullptr, v_lin ? r : ff};
-  p.b[1] = Operand{vu, nullptr, v_lin ? r : ff};
+  p.a[0] = Operand{xu, r};
+  p.a[1] = Operand{static_cast<const char*>(xu) + xu_bstride * esz, r};
+  p.b[0] = Operand{vg, v_lin ? r : ff};
+  p.b[1] = Operand{vu, v_lin ? r : ff};
   p.scale[0] = svg;
   p.scale[1] = svu;
   p.out = out;
@@ -423,8 +425,8 @@ int prefill_swiglu(const Common& c, int a_src, const void* xu, int64_t xu_bstrid
 int prefill_v(const Common& c, int a_src, const void* xu, const void* v, const float* sv, bool v_lin, int T, int r,
               int dout, bool vec, void* y) {
   GemmParams p{};
-  p.a[0] = Operand{xu, nullptr, r};
-  p.b[0] = Operand{v, nullptr, v_lin ? r : dout};
+  p.a[0] = Operand{xu, r};
+  p.b[0] = Operand{v, v_lin ? r : dout};
   p.scale[0] = sv;
   p.out = y;
   p.ldo = dout;
@@ -1390,6 +1392,95 @@ bool decode_ok(const Common& c, int64_t T, std::initializer_list<int64_t> dims, 
   return true;
 }
 
+// fp32 streaming stages take aligned dimensions (multiples of 8), with one
+// step's 32-bit offsets in range.
+bool f32_ok(const Common& c, int64_t T, std::initializer_list<int64_t> dims, bool vec) {
+  if (!c.f32 || !vec || T >= (int64_t)1 << 22) return false;
+  for (int64_t v : dims)
+    if (v % 8 || v >= (int64_t)1 << 22) return false;
+  return true;
+}
+
+// Token tiles a block (mt) and K splits of an fp32 stage by a cost model in
+// matrix cycles: rounds of blocks (one per CU) of K mt 8 cycles per branch
+// and split plus ~6000 for the launch's ramp and the in-block sums, and
+// ~5000 for meeting through slices.
+int f32_plan(int64_t M, int64_t K, int64_t ntiles, int br, int64_t area, int* ks, int* splits) {
+  int best_mt = 4;
+  double best = -1;
+  for (int mt : {4, 2, 1}) {
+    if (mt > 1 && M <= 8 * mt) continue;  // more rows of padding than of tokens
+    const int64_t tiles = ntiles * ((M + 16 * mt - 1) / (16 * mt));
+    for (int64_t s = 1; s <= 32; ++s) {
+      const int64_t k = ((K + s - 1) / s + 15) / 16 * 16, sp = (K + k - 1) / k;
+      if (s > 1 && (sp != s || k < 128 || tiles > kDlMaxTiles || tiles * sp * br * 16 * mt * kSfTileN * 4 > area)) continue;
+      const double cost = (double)((tiles * sp + 255) / 256) * ((double)(k * mt * 8 * br) + 6000.0) + (sp > 1 ? 5000.0 + 300.0 * sp : 0.0);
+      if (best < 0 || cost < best) {
+        best = cost;
+        best_mt = mt;
+        *ks = (int)k;
+        *splits = (int)sp;
+      }
+    }
+  }
+  return best_mt;
+}
+
+int f32_stage(const Common& c, int stage, int64_t M, int64_t K, int nseg, bool dual, const float* const* a,
+              const void* const* w, bool w_lin, const int64_t* N, float* const* out, const float* resid, char* ws,
+              const Ws& L, const char* what, bool a_t = false, bool out_t = false) {
+  StreamF32Params p{};
+  p.out_t = out_t;
+  p.M = (int)M;
+  // slices: the decode slice area up to kDlMaxT tokens, else y32 (unused on this path)
+  const bool small = M <= kDlMaxT;
+  p.slices = reinterpret_cast<float*>(ws + (small ? L.slices : L.y32));
+  const int64_t area = std::min<int64_t>((int64_t)(small ? L.need - L.slices : L.part - L.y32), 0x7ffffff0);
+  p.slice_bytes = (uint32_t)area;
+  for (int i = 0; i < nseg; ++i) p.tiles += !dual || i == 0 ? (int)((N[i] + kSfTileN - 1) / kSfTileN) : 0;
+  int ks = 0;
+  const int mt = f32_plan(M, K, p.tiles, dual ? 2 : 1, area, &ks, &p.splits);
+  p.mtiles = (int)((M + 16 * mt - 1) / (16 * mt));
+  p.sync = reinterpret_cast<uint64_t*>(ws + L.sync);
+  p.resid = resid;
+  for (int i = 0; i < nseg; ++i)
+    p.seg[i] = StreamF32Seg{a[i], static_cast<const float*>(w[i]), out[dual ? 0 : i], w_lin ? K : N[i], (int)K, (int)N[i],
+                            (int)((N[i] + kSfTileN - 1) / kSfTileN), ks};
+  const char* why = nullptr;
+  StageScope ss(stage, c.st);
+  return check(launch_stream_f32(p, mt, w_lin, dual, a_t, c.st, &why), what, why);
+}
+
+// The two halves of an fp32 layer: h = SiLU(x.ug.vg) * (x.uu.vu), y = a.u.v.
+int f32_gate_up(const Common& c, const void* x, const void* ug, const void* vg, const void* uu, const void* vu, bool u_lin,
+                bool v_lin, int64_t T, int64_t d, int64_t ff, int64_t r, void* h, char* ws, const Ws& L,
+                bool out_t = false) {
+  float* xu = reinterpret_cast<float*>(ws + L.xu32);
+  const float* a1[2] = {static_cast<const float*>(x), static_cast<const float*>(x)};
+  const void* w1[2] = {ug, uu};
+  const int64_t n1[2] = {r, r};
+  float* o1[2] = {xu, xu + T * r};
+  int rc = f32_stage(c, ST_GU_XU, T, d, 2, false, a1, w1, u_lin, n1, o1, nullptr, ws, L, "fp32 X.U");
+  if (rc) return rc;
+  const float* a2[2] = {xu, xu + T * r};
+  const void* w2[2] = {vg, vu};
+  const int64_t n2[2] = {ff, ff};
+  float* o2[1] = {static_cast<float*>(h)};
+  return f32_stage(c, ST_GU_XUV, T, r, 2, true, a2, w2, v_lin, n2, o2, nullptr, ws, L, "fp32 XU.V", false, out_t);
+}
+
+int f32_xuv(const Common& c, const void* a, const void* u, const void* v, bool u_lin, bool v_lin, int64_t T, int64_t din,
+            int64_t dout, int64_t r, void* y, const void* resid, char* ws, const Ws& L, bool a_t = false) {
+  float* xu = reinterpret_cast<float*>(ws + L.xu32) + 2 * T * r;
+  const float* a1 = static_cast<const float*>(a);
+  int rc = f32_stage(c, ST_D_XU, T, din, 1, false, &a1, &u, u_lin, &r, &xu, nullptr, ws, L, "fp32 h.Ud", a_t);
+  if (rc) return rc;
+  const float* a2 = xu;
+  float* o = static_cast<float*>(y);
+  return f32_stage(c, ST_D_XUV, T, r, 1, false, &a2, &v, v_lin, &dout, &o, static_cast<const float*>(resid), ws, L,
+                   "fp32 XUd.Vd");
+}
+
 // The persistent decode layer takes bf16 activations and factors in natural
 // layout, T <= kDlMaxT, ranks and d multiples of 128 and ff a multiple of 64
 // (its tiles), every operand below 2 GB (32-bit buffer offsets).
@@ -1908,7 +1999,10 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
     return check(launch_transpose_bf16(hn, ff, static_cast<uint16_t*>(h), T, (int)T, (int)ff, c.st), "h transpose");
   }
 
-  const Operand ax{x, nullptr, d};
+  if (f32_ok(c, T, {d, ff, r}, vec))
+    return f32_gate_up(c, x, ug, vg, uu, vu, u_lin, v_lin, T, d, ff, r, h, ws, L, out_t);
+
+  const Operand ax{x, d};
   const void* us[2] = {ug, uu};
   const float* sus[2] = {s_ug, s_uu};
   int a_src = 0;
@@ -1977,7 +2071,11 @@ int svdmlp_xuv(const void* x, const void* u, const void* v, const float* s_u, co
                  fp8 ? s_v : nullptr);
   }
 
-  const Operand ax{x, nullptr, x_t ? T : din};
+  if (f32_ok(c, T, {din, dout, r}, vec))
+    return f32_xuv(c, x, u, v, u_lin, v_lin, T, din, dout, r, y, nullptr, ws, L, x_t);
+
+  vec = vec && (!x_t || T % 8 == 0);
+  const Operand ax{x, x_t ? T : din};
   const void* us[1] = {u};
   const float* sus[1] = {s_u};
   int a_src = 0;
@@ -2215,7 +2313,15 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
     return big_v(c, reinterpret_cast<const uint16_t*>(ws + L.xu_bf16), vd, v_lin, T, r_d, d, ws, L, y, S[5], ld.vd);
   }
 
-  const Operand ax{x, nullptr, d};
+  if (f32_ok(c, T, {d, ff, r_gu, r_d}, vec)) {
+    void* hbuf = ws + L.h;
+    if ((rc = f32_gate_up(c, x, ug, vg, uu, vu, u_lin, v_lin, T, d, ff, r_gu, hbuf, ws, L))) return rc;
+    // the MLP block's residual add rides on the last stage's output
+    if (blk) blk->resid_done = true;
+    return f32_xuv(c, hbuf, ud, vd, u_lin, v_lin, T, ff, d, r_d, y, blk ? blk->x : nullptr, ws, L);
+  }
+
+  const Operand ax{x, d};
   const void* us[2] = {ug, uu};
   const float* sus[2] = {S[0], S[2]};
   int a_src = 0;
@@ -2226,7 +2332,7 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
   void* hbuf = ws + L.h;
   rc = prefill_swiglu(c, a_src, xu, xu_bs, vg, vu, S[1], S[3], v_lin, T, r_gu, ff, vec, false, hbuf);
   if (rc) return rc;
-  const Operand ah{hbuf, nullptr, ff};
+  const Operand ah{hbuf, ff};
   const void* ud1[1] = {ud};
   const float* sud[1] = {S[4]};
   rc = prefill_xu(c, ah, true, ud1, fp8 ? sud : nullptr, u_lin, T, ff, r_d, 1, vec, ws, L, 2, &a_src, &xu, &xu_bs);

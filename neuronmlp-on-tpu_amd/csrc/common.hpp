@@ -55,6 +55,16 @@ __device__ __forceinline__ float e4m3_to_f32(uint32_t b) {
   return __uint_as_float(s | ((e + 120u) << 23) | (m << 20));
 }
 
+// 8 fp8 e4m3fn values (bytes of v.x, then v.y) widened exactly to 8
+// bf16 packed in pairs (every e4m3 value, subnormals and NaN included, is a
+// bf16 value; the hardware conversion with scale 1 is exact).
+__device__ __forceinline__ u32x4 fp8x8_to_bf16x8(u32x2 v) {
+  return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.x, 1.0f, false)),
+               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.x, 1.0f, true)),
+               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.y, 1.0f, false)),
+               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.y, 1.0f, true))};
+}
+
 // Branch-stable SiLU in fp32 (kernels/reference.py:37-51): every exp
 // argument is <= 0, so 1 + z lies in [1, 2] and the hardware reciprocal
 // (v_rcp_f32, 1 ulp) stands in for an IEEE division, whose scale / fma /

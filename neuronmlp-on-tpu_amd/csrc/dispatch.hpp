@@ -53,6 +53,10 @@ hipError_t launch_big(const BigDesc& d, const BigParams& p, int splits, int batc
 // columns (cg 2: fp8 up to 32 tokens), dual the gate/up pair of a column tile.
 struct StreamParams;
 hipError_t launch_stream(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st, const char** why);
+// fp32 streaming stage (stream_f32.hpp): mt 16-row token tiles a block, at:
+// activations given as (K, M).
+struct StreamF32Params;
+hipError_t launch_stream_f32(const StreamF32Params& p, int mt, bool lin, bool dual, bool at, hipStream_t st, const char** why);
 hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t st);
 // MLP block prologue / epilogue: y = act(gain * rmsnorm(x)), y = act(x + y).
 hipError_t launch_rmsnorm(const void* x, const float* gain, void* y, int64_t T, int64_t d, float eps, bool bf16,

@@ -14,9 +14,9 @@
 //    (the reference's natural (in, out) weights) are loaded as 4(k) x 8(n)
 //    blocks with 16-byte global loads and transposed in registers before the
 //    LDS write; no extra HBM pass, no host-side transpose.
-//  * The A operand may be an fp32 workspace (split-K partial sums) or a pair
-//    of fp32 gate/up sums; it is rounded to bf16 on the way into LDS, which is
-//    exactly the rounding the reference applies at each GEMM boundary.
+//  * The A operand may be an fp32 workspace (split-K partial sums); it is
+//    rounded to bf16 on the way into LDS, which is exactly the rounding the
+//    reference applies at each GEMM boundary.
 //  * Two LDS stages: global loads for tile k+1 are in flight while tile k is
 //    multiplied; one barrier per K tile.
 //  * Epilogues: bf16 store, fp32 store, fp32 atomic add (split-K), and the
@@ -31,14 +31,13 @@
 
 namespace svdmlp {
 
-enum SrcKind : int { SRC_BF16 = 0, SRC_F32 = 1, SRC_FP8 = 2, SRC_SWIGLU = 3 };
+enum SrcKind : int { SRC_BF16 = 0, SRC_F32 = 1, SRC_FP8 = 2 };
 // EPI_STORE: plain store (bf16 or fp32 by OUT_F32); EPI_ATOMIC: fp32 atomic
 // add of a split-K partial; EPI_SWIGLU: out = silu(g) * u over two branches.
 enum EpiKind : int { EPI_STORE = 0, EPI_ATOMIC = 2, EPI_SWIGLU = 3 };
 
 struct Operand {
   const void* p;   // element (row, k) or (k, row) base pointer
-  const void* p2;  // SRC_SWIGLU: the "up" half (same layout as p)
   int64_t ld;      // leading dimension in elements
 };
 
@@ -74,12 +73,8 @@ __device__ __forceinline__ float load_elem_f32(const Operand& op, int64_t off) {
     return bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(op.p)[off]);
   } else if constexpr (SRC == SRC_F32) {
     return reinterpret_cast<const float*>(op.p)[off];
-  } else if constexpr (SRC == SRC_FP8) {
-    return e4m3_to_f32(reinterpret_cast<const uint8_t*>(op.p)[off]);
   } else {
-    const float g = reinterpret_cast<const float*>(op.p)[off];
-    const float u = reinterpret_cast<const float*>(op.p2)[off];
-    return silu_f32(g) * u;
+    return e4m3_to_f32(reinterpret_cast<const uint8_t*>(op.p)[off]);
   }
 }
 
@@ -95,28 +90,8 @@ __device__ __forceinline__ u32x4 load8_as_bf16(const Operand& op, int64_t off) {
     const f32x4 hi = *reinterpret_cast<const f32x4*>(f + 4);
     return u32x4{pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w),
                  pack_bf16x2(hi.x, hi.y), pack_bf16x2(hi.z, hi.w)};
-  } else if constexpr (SRC == SRC_FP8) {
-    const u32x2 w = ldg64(reinterpret_cast<const uint8_t*>(op.p) + off);
-    u32x4 r;
-    // e4m3 values are exact in bf16: take the top half of the fp32 value.
-    r.x = (__float_as_uint(e4m3_to_f32(w.x & 0xff)) >> 16) |
-          (__float_as_uint(e4m3_to_f32((w.x >> 8) & 0xff)) & 0xffff0000u);
-    r.y = (__float_as_uint(e4m3_to_f32((w.x >> 16) & 0xff)) >> 16) |
-          (__float_as_uint(e4m3_to_f32(w.x >> 24)) & 0xffff0000u);
-    r.z = (__float_as_uint(e4m3_to_f32(w.y & 0xff)) >> 16) |
-          (__float_as_uint(e4m3_to_f32((w.y >> 8) & 0xff)) & 0xffff0000u);
-    r.w = (__float_as_uint(e4m3_to_f32((w.y >> 16) & 0xff)) >> 16) |
-          (__float_as_uint(e4m3_to_f32(w.y >> 24)) & 0xffff0000u);
-    return r;
   } else {
-    const float* g = reinterpret_cast<const float*>(op.p) + off;
-    const float* u = reinterpret_cast<const float*>(op.p2) + off;
-    const f32x4 g0 = *reinterpret_cast<const f32x4*>(g), g1 = *reinterpret_cast<const f32x4*>(g + 4);
-    const f32x4 u0 = *reinterpret_cast<const f32x4*>(u), u1 = *reinterpret_cast<const f32x4*>(u + 4);
-    return u32x4{pack_bf16x2(silu_f32(g0.x) * u0.x, silu_f32(g0.y) * u0.y),
-                 pack_bf16x2(silu_f32(g0.z) * u0.z, silu_f32(g0.w) * u0.w),
-                 pack_bf16x2(silu_f32(g1.x) * u1.x, silu_f32(g1.y) * u1.y),
-                 pack_bf16x2(silu_f32(g1.z) * u1.z, silu_f32(g1.w) * u1.w)};
+    return fp8x8_to_bf16x8(ldg64(reinterpret_cast<const uint8_t*>(op.p) + off));
   }
 }
 

@@ -134,16 +134,6 @@ __device__ __forceinline__ u32x2 lds_read_tr8(lds_cptr p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((SVDMLP_LDS i32x2v*)(p)));
 }
 
-// 8 fp8 e4m3fn values (k order, bytes of v.x then v.y) widened exactly to 8
-// bf16 packed in pairs (every e4m3 value, subnormals and NaN included, is a
-// bf16 value; the hardware conversion with scale 1 is exact).
-__device__ __forceinline__ u32x4 fp8x8_to_bf16x8(u32x2 v) {
-  return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.x, 1.0f, false)),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.x, 1.0f, true)),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.y, 1.0f, false)),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.y, 1.0f, true))};
-}
-
 // bf16(a + b) of four bf16 pairs (the residual add of the MLP block).
 __device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b) {
   return pack_bf16x2(__uint_as_float(a << 16) + __uint_as_float(b << 16),

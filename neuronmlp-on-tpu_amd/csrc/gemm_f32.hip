@@ -1,24 +1,22 @@
 // fp32-MFMA GEMM instances (v_mfma_f32_16x16x4_f32): the reference's
-// mixed_precision=False / float32 arm, computed without any rounding to bf16.
+// mixed_precision=False / float32 arm, computed without any rounding to bf16,
+// for unaligned operands (the streaming stages of stream_f32.hpp take the
+// aligned ones).
 #include "dispatch.hpp"
 
 namespace svdmlp {
 
 namespace {
 
-template <int NBR, int EPI, bool AK, bool BK, bool OT, bool VEC>
+template <int NBR, int EPI, bool AK, bool BK, bool OT>
 hipError_t go(const GemmParams& p, int splits, int batch, hipStream_t st) {
-  using C = GemmCfg<kGemmBM, kGemmBN, 2, 2, float, SRC_F32, SRC_F32, AK, BK, NBR, EPI, OT, true, VEC>;
+  using C = GemmCfg<kGemmBM, kGemmBN, 2, 2, float, SRC_F32, SRC_F32, AK, BK, NBR, EPI, OT, true, false>;
   return run_gemm<C>(p, splits, batch, st);
 }
 
 template <int NBR, int EPI, bool AK, bool OT>
 hipError_t go2(const GemmDesc& d, const GemmParams& p, int splits, int batch, hipStream_t st) {
-  return expand_bool(d.b_kc, [&](auto bk) {
-    return expand_bool(d.vec, [&](auto vec) {
-      return go<NBR, EPI, AK, decltype(bk)::value, OT, decltype(vec)::value>(p, splits, batch, st);
-    });
-  });
+  return expand_bool(d.b_kc, [&](auto bk) { return go<NBR, EPI, AK, decltype(bk)::value, OT>(p, splits, batch, st); });
 }
 
 }  // namespace

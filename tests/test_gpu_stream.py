@@ -123,3 +123,39 @@ def test_stream_two_streams(gpu):
     torch.cuda.synchronize()
     for i in range(2):
         assert all(torch.equal(g.view(torch.int16), want[i].view(torch.int16)) for g in got[i])
+
+
+# fp32 stages (csrc/stream_f32.hpp).  Tolerance: a product over K terms summed
+# in fp32 is off by at most about sqrt(K) 2^-24 of its norm, 7e-6 at K = 14336
+# and less at these sizes; three products in a row and SiLU's reciprocal
+# (1 ulp) stay below 1e-5.
+@pytest.mark.parametrize("T", [1, 16, 17, 64, 65, 130, 300])
+@pytest.mark.parametrize("kind", ["natural", "linear"])
+@pytest.mark.parametrize("shape", [inputs.LayerShape(136, 200, 72, 40), inputs.LayerShape(1024, 3584, 256),
+                                   inputs.LayerShape(264, 1040, 392, 8)])
+def test_f32_stages(gpu, shape, kind, T):
+    x, f = inputs.make_layer(shape, T=T, seed=500 + T)
+    xt = torch.from_numpy(x).to(gpu)
+    ft = [torch.from_numpy(a).to(gpu) for a in f]
+    if kind == "linear":
+        ft = [a.t().contiguous().t() for a in ft]
+    w = [a.double() for a in ft]
+    g = (xt.double() @ w[0]) @ w[1]
+    h64 = g * torch.sigmoid(g) * ((xt.double() @ w[2]) @ w[3])
+    rel = lambda a, b: float((a.double() - b).norm() / b.norm())  # noqa: E731
+    h = ops.fused_gate_up(xt, *ft[:4])
+    assert rel(h, h64) < 1e-5
+    y = ops.fused_xuv(h, *ft[4:])
+    assert rel(y, (h.double() @ w[4]) @ w[5]) < 1e-5
+    out = ops.svd_mlp(xt, *ft)
+    assert rel(out, (h64 @ w[4]) @ w[5]) < 1e-5
+    assert torch.equal(ops.svd_mlp(xt, *ft), out)
+    # transposed operands: the same sums
+    if T % 8 == 0:
+        assert torch.equal(ops.fused_gate_up(xt, *ft[:4], out_transposed=True), h.t())
+        assert torch.equal(ops.fused_xuv(h.t().contiguous(), *ft[4:], x_transposed=True), y)
+    gain = torch.rand(shape.d, device=gpu) + 0.5
+    xn = xt.double() * torch.rsqrt(xt.double().pow(2).mean(1, keepdim=True) + 1e-5) * gain.double()
+    g = (xn @ w[0]) @ w[1]
+    want = xt.double() + ((g * torch.sigmoid(g) * ((xn @ w[2]) @ w[3])) @ w[4]) @ w[5]
+    assert rel(ops.svd_mlp_block(xt, gain, *ft), want) < 1e-5
