@@ -1950,9 +1950,9 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
   if (ws_bytes < L.need) return fail("workspace too small: need %zu bytes, got %zu", L.need, ws_bytes);
   const Common c{act_dtype, w_dtype, act_dtype == SVDMLP_F32, (hipStream_t)stream};
   const bool u_lin = flags & SVDMLP_U_LINEAR, v_lin = flags & SVDMLP_V_LINEAR, out_t = flags & SVDMLP_OUT_T;
-  bool vec = d % 8 == 0 && ff % 8 == 0 && r % 8 == 0 && (!out_t || T % 8 == 0);
+  bool vec = d % 8 == 0 && ff % 8 == 0 && r % 8 == 0;
   for (const void* q : {x, ug, vg, uu, vu, (const void*)h, (const void*)workspace}) vec = vec && aligned16(q);
-  if (fp8 && !vec) return fail("fp8 weights need d, ff and r to be multiples of 8 and 16-byte aligned buffers");
+  if (fp8 && (!vec || (out_t && T % 8))) return fail("fp8 weights need d, ff and r to be multiples of 8 and 16-byte aligned buffers");
   char* ws = static_cast<char*>(workspace);
 
   if (decode_ok(c, T, {d, ff, r}, vec)) {
@@ -1971,7 +1971,7 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
     const void* w[2] = {vg, vu};
     const float* s[2] = {s_vg, s_vu};
     const int64_t n[2] = {ff, ff};
-    const bool direct_t = out_t && stream_out_t_ok(T, ff, L, ws_bytes);
+    const bool direct_t = out_t && T % 8 == 0 && stream_out_t_ok(T, ff, L, ws_bytes);
     uint16_t* hn = out_t && !direct_t ? reinterpret_cast<uint16_t*>(ws + L.h) : static_cast<uint16_t*>(h);
     const StreamOut o[1] = {{hn, direct_t ? T : ff, direct_t}};
     if ((rc = stream_stage(c, ST_DEC_GU_XUV, T, r, 2, true, a, w, fp8 ? s : nullptr, v_lin, n, o, ws, L, ws_bytes, "decode XU.V")) ||
@@ -2002,6 +2002,7 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
   if (f32_ok(c, T, {d, ff, r}, vec))
     return f32_gate_up(c, x, ug, vg, uu, vu, u_lin, v_lin, T, d, ff, r, h, ws, L, out_t);
 
+  vec = vec && (!out_t || T % 8 == 0);  // 16-byte pieces of transposed rows
   const Operand ax{x, d};
   const void* us[2] = {ug, uu};
   const float* sus[2] = {s_ug, s_uu};
@@ -2031,9 +2032,9 @@ int svdmlp_xuv(const void* x, const void* u, const void* v, const float* s_u, co
   const Common c{act_dtype, w_dtype, act_dtype == SVDMLP_F32, (hipStream_t)stream};
   const bool u_lin = flags & SVDMLP_U_LINEAR, v_lin = flags & SVDMLP_V_LINEAR;
   bool x_t = flags & SVDMLP_X_T;
-  bool vec = din % 8 == 0 && dout % 8 == 0 && r % 8 == 0 && (!x_t || T % 8 == 0);
+  bool vec = din % 8 == 0 && dout % 8 == 0 && r % 8 == 0;
   for (const void* q : {x, u, v, (const void*)y, (const void*)workspace}) vec = vec && aligned16(q);
-  if (fp8 && !vec) return fail("fp8 weights need d_in, d_out and r to be multiples of 8 and 16-byte aligned buffers");
+  if (fp8 && (!vec || (x_t && T % 8))) return fail("fp8 weights need d_in, d_out and r to be multiples of 8 and 16-byte aligned buffers");
   char* ws = static_cast<char*>(workspace);
   // x given as (I, S) (the reference's TPU launcher fused_three_mm_XTUV,
   // test_speedup.py:500-519): bf16 x is transposed once into the workspace's

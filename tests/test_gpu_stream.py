@@ -64,7 +64,7 @@ def test_stream_entry_points(gpu, shape, kind, T):
     for _ in range(3):
         assert torch.equal(ops.fused_gate_up(xt, *ft[:4]).view(torch.int16), h.view(torch.int16))
         assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
-    if T % 8 == 0:  # transposed operands: the natural result's bits
+    if T % 8 == 0 or kind != "fp8":  # transposed operands (fp8: T % 8 == 0 only): the natural result's bits
         hT = ops.fused_gate_up(xt, *ft[:4], out_transposed=True)
         assert torch.equal(hT.view(torch.int16), h.t().contiguous().view(torch.int16))
         yT = ops.fused_xuv(h.t().contiguous(), *ft[4:], x_transposed=True)
@@ -105,6 +105,14 @@ def test_stream_after_a_timeout(gpu):
     assert torch.isnan(ops.svd_mlp(xt, *ft, workspace=ws)).all()
     assert ops.workspace_status(ws, reset=True) is True
     assert _rel(_np(ops.svd_mlp(xt, *ft, workspace=ws)), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+
+
+def test_fp8_transposed_odd_tokens_stay_refused(gpu):
+    _, _, xt, ft = _layer(inputs.LayerShape(264, 528, 136), 9, 14, "fp8", gpu)
+    for call in (lambda: ops.fused_gate_up(xt, *ft[:4], out_transposed=True),
+                 lambda: ops.fused_xuv(torch.zeros(528, 9, dtype=torch.bfloat16, device=gpu), *ft[4:], x_transposed=True)):
+        with pytest.raises(ValueError, match="multiples of 8"):
+            call()
 
 
 def test_stream_two_streams(gpu):
@@ -151,9 +159,8 @@ def test_f32_stages(gpu, shape, kind, T):
     assert rel(out, (h64 @ w[4]) @ w[5]) < 1e-5
     assert torch.equal(ops.svd_mlp(xt, *ft), out)
     # transposed operands: the same sums
-    if T % 8 == 0:
-        assert torch.equal(ops.fused_gate_up(xt, *ft[:4], out_transposed=True), h.t())
-        assert torch.equal(ops.fused_xuv(h.t().contiguous(), *ft[4:], x_transposed=True), y)
+    assert torch.equal(ops.fused_gate_up(xt, *ft[:4], out_transposed=True), h.t())
+    assert torch.equal(ops.fused_xuv(h.t().contiguous(), *ft[4:], x_transposed=True), y)
     gain = torch.rand(shape.d, device=gpu) + 0.5
     xn = xt.double() * torch.rsqrt(xt.double().pow(2).mean(1, keepdim=True) + 1e-5) * gain.double()
     g = (xn @ w[0]) @ w[1]
