@@ -480,6 +480,7 @@ struct Tune {
   // decode layer: most K splits of phases 1, 3, 4 (0: grid / tiles; -1: the
   // defaults, dls3 8 at two token tiles, dls4 4 at four, else grid / tiles)
   int dls1 = 0, dls3 = -1, dls4 = -1;
+  int p2k = -1;        // decode layer: smallest K of a phase-2 split (0: no splits, -1: p2_splits' own)
   bool dlpff = true;   // decode layer: the weight prefetch at a grid barrier fills the whole ring
   bool dlready = true;  // decode layer: phase 4 waits for its XU_d tiles' ready flags, not a grid barrier
   bool dlready3 = true; // ... also from two token tiles up (XU_d tiles written by all their splits)
@@ -566,6 +567,7 @@ const Tune& tune() {
         if (k == "kg") r.kg = v;
         if (k == "kgw") r.kgw = v;
         if (k == "kgs") r.kgs = v;
+        if (k == "p2k") r.p2k = v;
         if (k == "dls1") r.dls1 = v;
         if (k == "dls3") r.dls3 = v;
         if (k == "dls4") r.dls4 = v;
@@ -1537,6 +1539,24 @@ bool p2split_fits(int64_t d, int64_t ff, int64_t r_gu, int64_t r_d, int grid, in
   return ff % 128 == 0 && 2 * nt2 <= grid && (r_gu + r_u) / 128 + r_d / 128 + d / 128 + nt2 <= kDlMaxTiles;
 }
 
+// K splits of the one-branch phase-2 units: as many as fill the grid, each of
+// at least 256 k of the smaller rank (128 at eight token tiles, where a unit's
+// chunk takes longest).  Without them phase 2, half of the layer's bytes,
+// streams on 2 ff / 128 CUs.  us per layer, one box, no splits -> splits:
+// (3072, 8192, 1792) T=4 / 8 / 48 / 128 46.0 / 46.3 / 55.7 / 75.2 -> 43.1 /
+// 43.3 / 49.5 / 68.7, (4096, 1792, 1024) T=8 / 64 31.5 / 40.9 -> 27.9 / 35.4,
+// (2560, 6912, 1408) T=8 38.2 -> 35.4; at 128 tokens 256 k against 128:
+// (4096, 1792, 1024) 46.1 / 44.6, (1024, 3584, 256) 46.0 / 43.9.
+int p2_splits(int64_t T, int64_t d, int64_t ff, int64_t r_gu, int64_t r_d, int grid, int64_t r_u) {
+  const int64_t least = tune().p2k >= 0 ? tune().p2k : (T > 64 ? 128 : 256);
+  if (!p2split_fits(d, ff, r_gu, r_d, grid, r_u) || least == 0) return 1;
+  int64_t s = std::min(grid / (2 * (ff / 128)), std::min(r_gu, r_u) / least);
+  // every split of both branches has k of its own (K per split in whole 32-k chunks)
+  for (; s > 1; --s)
+    if ((s - 1) * (((r_gu + s - 1) / s + 31) / 32 * 32) < r_gu && (s - 1) * (((r_u + s - 1) / s + 31) / 32 * 32) < r_u) break;
+  return (int)std::max<int64_t>(1, s);
+}
+
 // r_u >= 0 and != r_gu: distinct gate and up ranks (the caller checked
 // decode_layer_ok and p2split_fits with both; phase 2 runs one-branch units).
 int decode_layer(const Common& c, const void* x, const void* ug, const void* vg, const void* uu, const void* vu,
@@ -1580,9 +1600,14 @@ int decode_layer(const Common& c, const void* x, const void* ug, const void* vg,
   // HBM channels, and 256-byte pieces spread them (T=4 / 8 / 16: 75.8 / 76.4
   // / 78.2 -> 73.2 / 73.5 / 75.0 us); with padded rows the pair's extra
   // slice round trip costs ~1 us there (T=8 69.3 -> 70.4 us).
-  const bool p2_pays = mt >= 2 || ld.dense;
+  // Narrow layers leave CUs idle there: their units also split K, as many
+  // ways as fill the grid (p2_splits).
+  const int s2 = contract ? 1 : p2_splits(T, d, ff, r_gu, r_d, grid, r_u);
+  const bool p2_pays = mt >= 2 || ld.dense || s2 > 1;
   p.p2split = !contract && p2split_fits(d, ff, r_gu, r_d, grid, r_u) &&
               (two || tune().p2split >= 2 || (tune().p2split == 1 && p2_pays));
+  p.p2s = p.p2split ? s2 : 1;
+  p.units2 *= p.p2s;
   // Phase 3 at two token tiles (17-32 tokens) in at most 8 K splits (176
   // units instead of 242 at the 8B shape): T=32 75.4-75.5 -> 74.8-74.9 us
   // padded, 79.7-79.8 -> 79.4-79.5 dense, T=17-24 0-0.6 us less; at four

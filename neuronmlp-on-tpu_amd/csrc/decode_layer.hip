@@ -69,11 +69,16 @@ hipError_t launch_decode_layer(const DecLayerParams& p, int mt, int grid, hipStr
     *why = "decode layer: the RMSNorm instance takes d <= 16384, a block per token and the block's buffers";
     return hipErrorInvalidValue;
   }
-  if (p.p2split && (contract || p.ff % 128 || p.units2 > grid || p.units2 != 2 * (p.ff / 128) ||
+  if (p.p2split && (contract || p.ff % 128 || p.units2 > grid || p.p2s < 1 || p.units2 != 2 * (p.ff / 128) * p.p2s ||
                     p.r_gu / 128 + p.r_up / 128 + p.r_d / 128 + p.d / 128 + p.ff / 128 > kDlMaxTiles)) {
     *why = "decode layer: one-branch phase 2 takes ff % 128 == 0, a block per unit and a counter per column tile";
     return hipErrorInvalidValue;
   }
+  for (int rk : {p.r_gu, p.r_up})
+    if (p.p2s != 1 && (!p.p2split || (p.p2s - 1) * (((rk + p.p2s - 1) / p.p2s + 31) / 32 * 32) >= rk)) {
+      *why = "decode layer: phase 2 in K splits takes one-branch units and a nonempty K range for each";
+      return hipErrorInvalidValue;
+    }
   if (p.r_up != p.r_gu && (!p.p2split || contract)) {
     *why = "decode layer: distinct gate and up ranks need the one-branch phase 2 (not the contracted layer)";
     return hipErrorInvalidValue;

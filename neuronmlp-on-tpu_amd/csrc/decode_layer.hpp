@@ -97,6 +97,10 @@ struct DecLayerParams {
   // counter after phases 1, 3 and 4's.  Otherwise a unit computes both over
   // 64 columns.
   int p2split;
+  // K splits of the one-branch units of phase 2 (1: none): unit u + s *
+  // (2 ff / 128) is split s of unit u, and the 2 p2s units of a column tile
+  // meet through its counter (dl_swiglu_split).
+  int p2s;
   // Phase 4 waits for its XU_d tiles' ready flags (kDlMaxFlags tiles at
   // most) instead of a grid barrier: the contracted layer, one token tile,
   // and from two tiles up with the tiles written by all their splits (dist).
@@ -708,6 +712,68 @@ __device__ __forceinline__ void dl_swiglu_pair_dist(const DlCtx& c, const DlUnit
     finish(std::integral_constant<int, HALF>{});
   else
     finish(std::integral_constant<int, 0>{});
+}
+
+// Phase 2 with the one-branch units split over K (DecLayerParams::p2s): the
+// 2 S units of a column tile (unit u % nu: branch u & 1 of tile (u % nu) / 2,
+// split u / nu) store their fp32 tiles as slice u and arrive on the tile's
+// counter.  At one token tile the last to arrive sums both branches' slices
+// in split order and writes h = bf16(SiLU(g) * u); from two tiles up (`dist`)
+// the others wait for it (dl_wait_reset) and each writes its share of the
+// tile, the same sums in the same order.
+template <int MT>
+__device__ __forceinline__ void dl_swiglu_split(const DlCtx& c, const DlUnit& U, const f32x4 (&acc)[MT], int u, int S,
+                                                int nu, uint32_t* cnt, float* slices, int* flag, uint16_t* h, bool dist,
+                                                uint64_t* sync, uint32_t spin, int* bad) {
+  const __amdgpu_buffer_rsrc_t rs = dl_slice_rsrc<MT>(slices);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const uint32_t off = 16 * mt + c.lr < c.T ? (uint32_t)(((u * MT + mt) * 2048 + 4 * threadIdx.x) * 4) : kDlPastSlices;
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(acc[mt].x), __float_as_uint(acc[mt].y),
+                                                 __float_as_uint(acc[mt].z), __float_as_uint(acc[mt].w)},
+                                           rs, off, 0, kDlSc1);
+  }
+  dl_wait_vm<0>();
+  dl_block_sync();
+  if (threadIdx.x == 0) *flag = dl_arrive_wrap(cnt, 2 * S);
+  dl_block_sync();
+  if (!*flag) {
+    if (!dist) return;
+    if (threadIdx.x == 0) dl_wait_reset(cnt, sync, spin, bad);
+    dl_block_sync();
+  }
+  constexpr int TOTAL = MT * 512;  // float4 elements of a tile
+  const int part = dist ? (u & 1) + 2 * (u / nu) : 0;
+  const int share = dist ? (TOTAL + 2 * S - 1) / (2 * S) : TOTAL;
+  const int e1 = min(TOTAL, (part + 1) * share), u0 = u % nu & ~1;
+  constexpr int SB = 4;  // splits in flight
+  for (int e = part * share + (int)threadIdx.x; e < e1; e += kDlThreads) {
+    const int mt = e >> 9, t = e & 511;  // element e: the lane t of block mt in every slice
+    const int m = 16 * mt + (t & 15);
+    if (m >= c.T) continue;
+    f32x4 v[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    for (int s0 = 0; s0 < S; s0 += SB) {
+      u32x4 x[SB][2];
+#pragma unroll
+      for (int i = 0; i < SB; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          x[i][b] = __builtin_amdgcn_raw_buffer_load_b128(
+              rs, s0 + i < S ? (uint32_t)((((u0 + b + (s0 + i) * nu) * MT + mt) * 2048 + 4 * t) * 4) : kDlPastSlices, 0,
+              kDlSc1);
+#pragma unroll
+      for (int i = 0; i < SB; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          v[b] += f32x4{__uint_as_float(x[i][b].x), __uint_as_float(x[i][b].y), __uint_as_float(x[i][b].z),
+                        __uint_as_float(x[i][b].w)};
+    }
+    const int w = t >> 6;
+    const int n = U.n0 + 64 * (w >> 2) + 16 * (w & 3) + 4 * ((t & 63) >> 4);
+    dl_store8(h + (int64_t)m * U.ldo + n,
+              u32x2{dl_pack_bf16x2(silu_f32(v[0].x) * v[1].x, silu_f32(v[0].y) * v[1].y),
+                    dl_pack_bf16x2(silu_f32(v[0].z) * v[1].z, silu_f32(v[0].w) * v[1].w)});
+  }
 }
 
 // Split-K combination of unit u = tile + split * nt (splits per tile) into
@@ -1369,9 +1435,16 @@ __global__ __launch_bounds__(kDlThreads, 1) void decode_layer_kernel(DecLayerPar
       U.ke = min(p.d, U.kb + p.ks1);
       U.dst = p.xu16 + (br ? (int64_t)T * p.r_gu : 0);
       U.ldo = br ? p.r_up : p.r_gu;
-    } else if (phase == 2 && p.p2split) {
+    } else if (!CONTRACT && phase == 2 && p.p2split) {
       // each branch over its own rank
       const int br = u & 1, rk = br ? p.r_up : p.r_gu;
+      int sp = 0, ks = rk;
+      if (p.p2s > 1) {
+        const int nu = p.ff / 64;
+        sp = u / nu;
+        u -= sp * nu;
+        ks = ((rk + p.p2s - 1) / p.p2s + 31) / 32 * 32;
+      }
       U.a0 = U.a1 = p.xu16 + (br ? (int64_t)T * p.r_gu : 0);
       U.lda = rk;
       U.a_bytes = (uint32_t)((int64_t)T * rk * 2);
@@ -1379,8 +1452,8 @@ __global__ __launch_bounds__(kDlThreads, 1) void decode_layer_kernel(DecLayerPar
       U.ldb = br ? p.ld_vu : p.ld_v;
       U.b_bytes = (uint32_t)((int64_t)rk * U.ldb * 2);
       U.n0 = (u >> 1) * 128;
-      U.kb = 0;
-      U.ke = rk;
+      U.kb = sp * ks;
+      U.ke = min(rk, U.kb + ks);
       U.dst = p.h;
       U.ldo = p.ff;
     } else if (phase == 2) {  // both branches of 64 columns: one rank (r_up == r_gu), one V pitch
@@ -1585,21 +1658,25 @@ __global__ __launch_bounds__(kDlThreads, 1) void decode_layer_kernel(DecLayerPar
       wait_xu(u & 1);
       f32x4 acc[MT];
       dl_run<MT, false>(c, U, u == b, acc);
-      uint32_t* pcnt = dl_tile_counter(p.sync, nt1 + nt3 + nt4 + (u >> 1));
+      uint32_t* pcnt = dl_tile_counter(p.sync, nt1 + nt3 + nt4 + U.n0 / 128);
+      float* const bank = p.slices + kDlBank24<MT> * kDlMaxGrid * MT * 2048;
       if constexpr (MT >= 2) {
         if (p.dist) {
-          dl_swiglu_pair_dist<MT>(c, U, acc, u, pcnt, p.slices + kDlBank24<MT> * kDlMaxGrid * MT * 2048, flag, p.h,
-                                  p.sync, spin_lds ? *spin_lds : spin, bad);
+          if (p.p2s > 1)
+            dl_swiglu_split<MT>(c, U, acc, u, p.p2s, p.ff / 64, pcnt, bank, flag, p.h, true, p.sync,
+                                spin_lds ? *spin_lds : spin, bad);
+          else
+            dl_swiglu_pair_dist<MT>(c, U, acc, u, pcnt, bank, flag, p.h, p.sync, spin_lds ? *spin_lds : spin, bad);
           if (h_epoch) {
             // count down on the phase-3 K splits whose columns this pair's h
-            // covers (both units of a pair write h); the last of a split
+            // covers (all units of a column tile write h); the last of a split
             // sets its flag
             dl_wait_vm<0>();
             dl_block_sync();
             if (threadIdx.x == 0) {
               for (int s = U.n0 / p.ks3; s < p.splits3 && s * p.ks3 < U.n0 + 128; ++s) {
                 const int kb = s * p.ks3, ke = min(p.ff, kb + p.ks3);
-                if (dl_arrive_wrap(dl_tile_counter(p.sync, p.hc0 + s), 2 * ((ke - 1) / 128 - kb / 128 + 1)))
+                if (dl_arrive_wrap(dl_tile_counter(p.sync, p.hc0 + s), 2 * p.p2s * ((ke - 1) / 128 - kb / 128 + 1)))
                   __hip_atomic_store(dl_ready_flag(p.sync, p.hf0 + s), h_epoch, __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_AGENT);
               }
@@ -1608,7 +1685,11 @@ __global__ __launch_bounds__(kDlThreads, 1) void decode_layer_kernel(DecLayerPar
           continue;
         }
       }
-      dl_swiglu_pair<MT>(c, U, acc, u, pcnt, p.slices + kDlBank24<MT> * kDlMaxGrid * MT * 2048, flag, p.h);
+      if (p.p2s > 1)
+        dl_swiglu_split<MT>(c, U, acc, u, p.p2s, p.ff / 64, pcnt, bank, flag, p.h, false, p.sync,
+                            spin_lds ? *spin_lds : spin, bad);
+      else
+        dl_swiglu_pair<MT>(c, U, acc, u, pcnt, bank, flag, p.h);
     }
   } else {
   // ---- phase 2: h = bf16(SiLU(XU_g . Vg) * (XU_u . Vu)) ----

@@ -166,3 +166,27 @@ def test_f32_stages(gpu, shape, kind, T):
     g = (xn @ w[0]) @ w[1]
     want = xt.double() + ((g * torch.sigmoid(g) * ((xn @ w[2]) @ w[3])) @ w[4]) @ w[5]
     assert rel(ops.svd_mlp_block(xt, gain, *ft), want) < 1e-5
+
+
+# The persistent decode layer's phase 2 in K splits (layers narrower than the
+# grid): 2 (3B-like ratio) and 9 (ff = 1792, rank 2304) ways, distinct gate and
+# up ranks whose splits end apart, the last-arrival (up to 16 tokens) and the
+# shared form, and eight token tiles (phase 3 on its K splits' h flags).
+@pytest.mark.parametrize("T", [4, 16, 17, 48, 100, 128])
+@pytest.mark.parametrize("ranks", [(512, 512, 256), (2304, 1152, 384)])
+@pytest.mark.parametrize("d,ff", [(1024, 8192), (512, 1792)])
+def test_decode_layer_phase2_splits(gpu, d, ff, ranks, T):
+    rng = np.random.default_rng(T + ff)
+    rg, ru, rd = ranks
+    mats = [inputs.random_matrix(rng, *s) for s in ((d, rg), (rg, ff), (d, ru), (ru, ff), (ff, rd), (rd, d))]
+    wide = [inputs.as_float32(a, torch.bfloat16) for a in mats]
+    xb = inputs.as_float32(rng.normal(size=(T, d)).astype(np.float32), torch.bfloat16)
+    xt, ft = inputs.to_torch(xb, torch.bfloat16, gpu), [inputs.to_torch(a, torch.bfloat16, gpu) for a in wide]
+    want = O.svd_mlp_ref(xb, *wide, dtype="bfloat16")
+    ops.clear_workspace_cache()
+    out = ops.svd_mlp(xt, *ft)
+    assert _rel(_np(out), want) < TOL
+    for _ in range(3):
+        assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
+    (ws,) = ops._WS_CACHE.values()
+    assert not any(ws[2560:4096].view(torch.int32).cpu().tolist()) and not ops.workspace_status()
