@@ -463,6 +463,7 @@ struct Tune {
   bool xutail = true;  // gate/up X.U with 1-2 rounds of tiles: one round without a split, the rest split
   bool gufuse = true;  // split gate/up XU.V passes: one reduction from both passes' slices
   bool gudual = true;  // gate/up XU.V passes in one launch (each block its g tile or split, then its u one)
+  bool gupair = true;  // split gate/up XU.V passes: the branches as batch entries with half the splits each
   bool gukg = true;    // ... split and at most 128 token rows: 128 x 128 K-group tiles
   int gukgu = 2;       // ... unsplit on 128 x 128 K-group tiles: 1 at 129-256 token rows, 2 while they fit one round
   int dlmin = 1 << 30; // lowest T for the persistent decode layer (min with kDlMinT)
@@ -556,6 +557,7 @@ const Tune& tune() {
         if (k == "xutail") r.xutail = v != 0;
         if (k == "gufuse") r.gufuse = v != 0;
         if (k == "gudual") r.gudual = v != 0;
+        if (k == "gupair") r.gupair = v != 0;
         if (k == "gukg") r.gukg = v != 0;
         if (k == "gukgu") r.gukgu = v;
         if (k == "dlmin") r.dlmin = v;
@@ -1041,11 +1043,12 @@ int big_xu(const Common& c, int stage, const void* a, int64_t lda, int64_t a_byt
 // h_blk (optional): asks for h in 16 x 16 block-major order (the fused
 // layer's h.Ud stage reads it so: BigParams::a_blk) and reports whether the
 // pass wrote it so (the split passes at one or two row tiles write
-// row-major h).
+// row-major h).  out_T (optional): the caller wants h as (ff, T) there; the
+// split passes' reduction writes it so, and *wrote_T says whether it did.
 int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, const void* vg, const void* vu,
                bool v_lin, int T, int r, int ff, uint16_t* gbuf, void* out, float* part, int64_t part_cap,
                const float* s_vg = nullptr, const float* s_vu = nullptr, int64_t ldv = 0, int r_u = 0,
-               int64_t ldv_u = 0, bool* h_blk = nullptr) {
+               int64_t ldv_u = 0, bool* h_blk = nullptr, void* out_T = nullptr, bool* wrote_T = nullptr) {
   const bool want_blk = h_blk && *h_blk && ff % 16 == 0;
   if (h_blk) *h_blk = false;
   if (r_u <= 0) r_u = r;
@@ -1109,7 +1112,22 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     const bool fused = tune().gufuse && (int64_t)(splits + splits_u) * per * 4 <= part_cap;
     float* upart = fused ? part + (int64_t)splits * per : part;
     int rc;
-    if (fused && tune().gudual && splits == splits_u && !v_lin) {
+    // An even number of splits as half as many per branch, the branches side
+    // by side as batch entries: the same blocks and K a block, half the fp32
+    // slices written and summed, and one pipeline fill a block instead of
+    // two.  us, one box, a g and a u split in every block -> a branch a block:
+    // 8B gate/up at 65 / 128 tokens 71.4 / 76.5 -> 64.7 / 71.4, 3B 48.6 / 49.3
+    // -> 39.8 / 39.9; 8B layer at 512 tokens 230 -> 212, with Linear factors at
+    // 128 / 512 170 / 247 -> 159 / 224, with fp8 ones at 256 187 -> 175.
+    if (fused && tune().gupair && nsp % 2 == 0 && r == r_u && ldb == ldb_u) {
+      const int ksb = nsp == 2 ? r : (r / (nsp / 2) + kq - 1) / kq * kq;
+      splits = splits_u = (r + ksb - 1) / ksb;
+      upart = part + (int64_t)splits * per;
+      rc = big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 2, fn, BEPI_STORE,
+                    ksb, part, ff, (int64_t)splits * per, nullptr, true, per, s_vg, s_vu, 0, 1, nullptr, nullptr,
+                    kg2 ? 2 : 1);
+      if (rc) return rc;
+    } else if (fused && tune().gudual && splits == splits_u && !v_lin) {
       // both passes' slices from one launch: every block its g split, then
       // its u split of the same tile
       const DualEntry du{r_u, xuu_bytes, r_u, ldb_u, vu_bytes, ks_u};
@@ -1131,10 +1149,12 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     }
     StageScope fin(ST_FINALIZE, c.st);
     const int mt = (T + bm - 1) / bm;
-    return check(launch_reduce_frag_bf16(upart, splits_u, per, per, static_cast<uint16_t*>(out), ff, (int64_t)T * ff,
-                                         T, ff, mt, (int)(per / ((int64_t)bm * mt) / (32 * fn)), fn,
+    const bool tr = out_T && T % 8 == 0;
+    if (wrote_T) *wrote_T = tr;
+    return check(launch_reduce_frag_bf16(upart, splits_u, per, per, static_cast<uint16_t*>(tr ? out_T : out), tr ? T : ff,
+                                         (int64_t)T * ff, T, ff, mt, (int)(per / ((int64_t)bm * mt) / (32 * fn)), fn,
                                          kg2 ? 8 : big_nw(fn, BEPI_STORE, v_lin), 1, c.st, fused ? nullptr : gbuf,
-                                         nullptr, kg2 ? 2 : 1, fused ? part : nullptr, fused ? splits : 0),
+                                         nullptr, kg2 ? 2 : 1, fused ? part : nullptr, fused ? splits : 0, tr),
                  "split-K SwiGLU reduce");
   }
   if (tune().gudual && (fn == 4 || fn == 7 || fn == 8) && !v_lin) {
@@ -2013,12 +2033,15 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
     const uint16_t* xu = reinterpret_cast<const uint16_t*>(ws + L.xu_bf16);
     uint16_t* gbuf = reinterpret_cast<uint16_t*>(ws + L.g);
     // (I, S) output (the reference's TPU launcher fused_mlp_up_T,
-    // test_speedup.py:522-544): h in the natural layout into the workspace's
-    // h region, then one transpose pass into the caller's buffer
+    // test_speedup.py:522-544): written by the split passes' reduction, else h
+    // in the natural layout into the workspace's h region, then one transpose
+    // pass into the caller's buffer
     uint16_t* hn = out_t ? reinterpret_cast<uint16_t*>(ws + L.h) : static_cast<uint16_t*>(h);
+    bool wrote_T = false;
     if ((rc = big_swiglu(c, xu, xu + T * r, vg, vu, v_lin, T, r, ff, gbuf, hn, reinterpret_cast<float*>(ws + L.part),
-                         (int64_t)(L.norm - L.part), fp8 ? s_vg : nullptr, fp8 ? s_vu : nullptr)) ||
-        !out_t)
+                         (int64_t)(L.norm - L.part), fp8 ? s_vg : nullptr, fp8 ? s_vu : nullptr, 0, 0, 0, nullptr,
+                         out_t ? h : nullptr, &wrote_T)) ||
+        !out_t || wrote_T)
       return rc;
     StageScope fin(ST_FINALIZE, c.st);
     return check(launch_transpose_bf16(hn, ff, static_cast<uint16_t*>(h), T, (int)T, (int)ff, c.st), "h transpose");

@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void reduce_frag_bf16_kernel(const float* in, 
                                                                int64_t bstride, uint16_t* out, int64_t ldo,
                                                                int64_t obstride, int M, int N, int mtiles, int nw,
                                                                const uint16_t* gate, const uint16_t* resid,
-                                                               const float* gsl, int gsplits) {
+                                                               const float* gsl, int gsplits, int out_t) {
   // tiles of (nw / 2) x 2 wave tiles: 256 rows (8 waves of 64, 4 of 128) or
   // 128 (the K-group tiles' four wave tiles of 64)
   constexpr int ROWS = 16 * FM, COLS = 16 * FN, PITCH = COLS + 8;  // staged row pitch (elements)
@@ -149,6 +149,18 @@ __global__ __launch_bounds__(256) void reduce_frag_bf16_kernel(const float* in, 
   }
   __syncthreads();
   uint16_t* dst = out + (int64_t)zb * obstride;
+  if (out_t) {  // (N, M): 8 rows of a column a lane, whole 128-byte pieces of an output row (M % 8 == 0)
+    for (int k = threadIdx.x; k < COLS * (ROWS / 8); k += 256) {
+      const int r = 8 * (k % (ROWS / 8)), c = k / (ROWS / 8);
+      if (m0 + r >= M || n0 + c >= N) continue;
+      const uint16_t* e = tile + r * PITCH + c;
+      u32x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = (uint32_t)e[2 * i * PITCH] | (uint32_t)e[(2 * i + 1) * PITCH] << 16;
+      *reinterpret_cast<u32x4*>(dst + (int64_t)(n0 + c) * ldo + m0 + r) = o;
+    }
+    return;
+  }
   for (int k = threadIdx.x; k < ROWS * (COLS / 8); k += 256) {
     const int r = k / (COLS / 8), c = 8 * (k % (COLS / 8));
     const int m = m0 + r, n = n0 + c;
@@ -166,9 +178,9 @@ __global__ __launch_bounds__(256) void reduce_frag_bf16_kernel(const float* in, 
 template <int FM, int FN>
 hipError_t go_reduce(const float* in, int splits, int64_t sstride, int64_t bstride, uint16_t* out, int64_t ldo,
                      int64_t obstride, int M, int N, int mtiles, int ntiles, int nw, int batch, const uint16_t* gate,
-                     const uint16_t* resid, hipStream_t st, const float* gsl, int gsplits) {
+                     const uint16_t* resid, hipStream_t st, const float* gsl, int gsplits, int out_t) {
   hipLaunchKernelGGL((reduce_frag_bf16_kernel<FM, FN>), dim3(mtiles * ntiles * nw, batch), dim3(256), 0, st, in,
-                     splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, nw, gate, resid, gsl, gsplits);
+                     splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, nw, gate, resid, gsl, gsplits, out_t);
   return hipGetLastError();
 }
 
@@ -177,20 +189,21 @@ hipError_t go_reduce(const float* in, int splits, int64_t sstride, int64_t bstri
 hipError_t launch_reduce_frag_bf16(const float* in, int splits, int64_t sstride, int64_t bstride, uint16_t* out,
                                    int64_t ldo, int64_t obstride, int M, int N, int mtiles, int ntiles, int fn, int nw,
                                    int batch, hipStream_t st, const uint16_t* gate, const uint16_t* resid, int kg,
-                                   const float* gsl, int gsplits) {
+                                   const float* gsl, int gsplits, int out_t) {
+  if (out_t && (M % 8 || resid || batch != 1)) return hipErrorInvalidValue;
   if (kg == 2) {  // 128-row K-group tiles: four 64-row wave tiles per tile
     if (nw != 8) return hipErrorInvalidValue;
-    if (fn == 4) return go_reduce<4, 4>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, 4, batch, gate, resid, st, gsl, gsplits);
-    if (fn == 6) return go_reduce<4, 6>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, 4, batch, gate, resid, st, gsl, gsplits);
+    if (fn == 4) return go_reduce<4, 4>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, 4, batch, gate, resid, st, gsl, gsplits, out_t);
+    if (fn == 6) return go_reduce<4, 6>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, 4, batch, gate, resid, st, gsl, gsplits, out_t);
     return hipErrorInvalidValue;
   }
   if (kg != 1) return hipErrorInvalidValue;
-  if (nw == 8 && fn == 8) return go_reduce<4, 8>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits);
-  if (nw == 8 && fn == 7) return go_reduce<4, 7>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits);
-  if (nw == 8 && fn == 6) return go_reduce<4, 6>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits);
-  if (nw == 8 && fn == 4) return go_reduce<4, 4>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits);
-  if (nw == 4 && fn == 4) return go_reduce<8, 4>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits);
-  if (nw == 4 && fn == 8) return go_reduce<8, 8>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits);
+  if (nw == 8 && fn == 8) return go_reduce<4, 8>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits, out_t);
+  if (nw == 8 && fn == 7) return go_reduce<4, 7>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits, out_t);
+  if (nw == 8 && fn == 6) return go_reduce<4, 6>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits, out_t);
+  if (nw == 8 && fn == 4) return go_reduce<4, 4>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits, out_t);
+  if (nw == 4 && fn == 4) return go_reduce<8, 4>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits, out_t);
+  if (nw == 4 && fn == 8) return go_reduce<8, 8>(in, splits, sstride, bstride, out, ldo, obstride, M, N, mtiles, ntiles, nw, batch, gate, resid, st, gsl, gsplits, out_t);
   return hipErrorInvalidValue;
 }
 
