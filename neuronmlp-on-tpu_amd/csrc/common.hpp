@@ -65,15 +65,16 @@ __device__ __forceinline__ u32x4 fp8x8_to_bf16x8(u32x2 v) {
                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v.y, 1.0f, true))};
 }
 
-// Branch-stable SiLU in fp32 (kernels/reference.py:37-51): every exp
-// argument is <= 0, so 1 + z lies in [1, 2] and the hardware reciprocal
-// (v_rcp_f32, 1 ulp) stands in for an IEEE division, whose scale / fma /
-// fixup sequence made the SwiGLU epilogue of the 8B layer ~4 us slower; the
-// result is rounded to bf16 (8 bits of mantissa) afterwards.
+// SiLU in fp32 (kernels/reference.py:37-51) as x / (1 + exp(-x)): six
+// instructions, two of them transcendental.  No branch is needed for large
+// negative x: exp(-x) overflows to infinity, whose reciprocal is 0, and x * 0
+// is the limit; 1 + exp(-x) >= 1 has the relative error of one rounding on
+// either side.  The hardware reciprocal (v_rcp_f32, 1 ulp) stands in for an
+// IEEE division, whose scale / fma / fixup sequence made the SwiGLU epilogue
+// of the 8B layer ~4 us slower; the result is rounded to bf16 (8 bits of
+// mantissa) afterwards, or is fp32 with the reciprocal's 1 ulp.
 __device__ __forceinline__ float silu_f32(float x) {
-  const float z = __expf(-fabsf(x));
-  const float r = __builtin_amdgcn_rcpf(1.0f + z);
-  return x * ((x >= 0.0f) ? r : z * r);
+  return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x));
 }
 
 // ---------------------------------------------------------------------------
