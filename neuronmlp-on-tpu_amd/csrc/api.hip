@@ -604,6 +604,26 @@ bool big_ok(const Common& c, bool vec, std::initializer_list<int64_t> bytes, std
   return true;
 }
 
+// A rank as the large-tile path holds XU: `p` columns, r itself where it is
+// whole 32-k stages, else rounded up to 64 with the map of BigParams::nmap.
+struct Rank {
+  int p;
+  RankMap map;
+};
+
+Rank big_rank(int64_t r) {
+  if (r % 32 == 0) return Rank{(int)r, RankMap{}};
+  const int64_t rp = (r + 63) / 64 * 64;
+  return Rank{(int)rp, RankMap{(int)(rp - 64), (int)(rp - r)}};
+}
+
+// ... takes ranks in whole 32-k stages, and others of at least one 64-wide
+// block in whole DMA pieces (8 bf16 or 16 fp8 columns).  XU's wider rows
+// (at most twice r) run on into the xu32 region after it.
+bool big_rank_ok(const Common& c, int64_t r) {
+  return r % 32 == 0 || (r >= 64 && r % (c.wt == SVDMLP_FP8_E4M3 ? 16 : 8) == 0);
+}
+
 // Waves per block of a large-tile launch: 4 only for the fn-8 natural-layout
 // store stages under SVDMLP_TUNE=nw=4.
 int big_nw(int fn, int epi, bool b_kc) { return (fn == 8 && epi == BEPI_STORE && !b_kc && tune().nw == 4) ? 4 : 8; }
@@ -634,8 +654,10 @@ int big_gemm(const Common& c, int stage, const void* a0, const void* a1, int64_t
              bool out_f32 = false, int64_t out_sstride = 0, const float* s0 = nullptr, const float* s1 = nullptr,
              int gfrag = 0, int out_frag = 0, const Entry1* e1 = nullptr, const uint16_t* resid = nullptr,
              int kg = 1, int out_blk = 0, int a_blk = 0, int tile0 = 0, int tiles = 0,
-             const DualEntry* du = nullptr) {
+             const DualEntry* du = nullptr, const RankMap& nmap = RankMap{}, const RankMap& kmap = RankMap{}) {
   BigParams p{};
+  p.nmap[0] = p.nmap[1] = nmap;  // ranks off the stages are the same for both entries
+  p.kmap[0] = p.kmap[1] = kmap;
   p.tile0 = tile0;
   p.tiles = tiles;
   p.out_blk = out_blk;
@@ -981,13 +1003,17 @@ int big_xu2(const Common& c, int stage, const void* a, int64_t lda, int64_t a_by
 // too few output tiles for the chip, K is split: each split writes an fp32
 // slice (plain stores) and one pass sums the slices in order into bf16.
 // a_blk: A (h of the fused layer) is 16 x 16 block-major (BigParams::a_blk).
+// Ranks off the 32-k stages are written big_rank(r).p columns wide (batch
+// stride T * p).
 int big_xu(const Common& c, int stage, const void* a, int64_t lda, int64_t a_bytes, const void* const* u, bool u_lin,
-           int T, int K, int r, int batch, char* ws, const Ws& L, const float* const* su = nullptr,
+           int T, int K, int r_in, int batch, char* ws, const Ws& L, const float* const* su = nullptr,
            int64_t ldu = 0, bool a_blk = false) {
+  const Rank rk = big_rank(r_in);
+  const int r = rk.p;  // columns of XU
   if (a_blk) a_bytes = (int64_t)((T + 15) / 16 * 16) * K * 2;  // whole 16-row blocks
   const int fn1 = stage == ST_GU_XU ? gate_xu_fn(T, K, r, batch) : down_xu_fn(T, K, r);
   const RankPlan pl = plan_rank(T, K, r, fn1, batch, -1, !u_lin && c.wt == SVDMLP_BF16, stage);
-  if (stage == ST_GU_XU && batch == 2 && !a_blk) {  // the split tail runs in the two-entry form
+  if (stage == ST_GU_XU && batch == 2 && !a_blk && r == r_in) {  // the split tail runs in the two-entry form
     double plain = 0.0;
     plan_ksplit(T, K, r, pl.fn, 2, -1, &plain, pl.kg);
     int tail_ks = K;
@@ -1006,22 +1032,22 @@ int big_xu(const Common& c, int stage, const void* a, int64_t lda, int64_t a_byt
     }
   }
   uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
-  const int64_t ldb = u_lin ? K : (ldu ? ldu : r);  // natural U may carry padded rows
-  const int64_t u_bytes = (int64_t)(u_lin ? r : K) * ldb * wbytes(c);
+  const int64_t ldb = u_lin ? K : (ldu ? ldu : r_in);  // natural U may carry padded rows
+  const int64_t u_bytes = (int64_t)(u_lin ? r_in : K) * ldb * wbytes(c);
   const void* u1 = batch > 1 ? u[1] : u[0];
   const float* s0 = su ? su[0] : nullptr;
   const float* s1 = su && batch > 1 ? su[1] : s0;
   if (splits == 1)
     return big_gemm(c, stage, a, a, lda, a_bytes, u[0], u1, ldb, u_bytes, u_lin, T, r, K, batch, fn,
                     BEPI_STORE, K, xu, r, (int64_t)T * r, nullptr, false, 0, s0, s1, 0, 0, nullptr, nullptr, kg, 0,
-                    a_blk);
+                    a_blk, 0, 0, nullptr, rk.map);
   float* part = reinterpret_cast<float*>(ws + L.part);
   const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, u_lin);
   if (kg == 2 || big_frag_reduce_ok(fn, nw)) {
     // slices in fragment order: per split, `batch` blocks of whole tiles
     const int64_t tp = (T + bm - 1) / bm * bm, np = ((int64_t)r + 32 * fn - 1) / (32 * fn) * (32 * fn), per = tp * np;
     int rc = big_gemm(c, stage, a, a, lda, a_bytes, u[0], u1, ldb, u_bytes, u_lin, T, r, K, batch, fn, BEPI_STORE, ks,
-                      part, r, per, nullptr, true, batch * per, s0, s1, 0, 1, nullptr, nullptr, kg, 0, a_blk);
+                      part, r, per, nullptr, true, batch * per, s0, s1, 0, 1, nullptr, nullptr, kg, 0, a_blk, 0, 0, nullptr, rk.map);
     if (rc) return rc;
     StageScope fin(ST_FINALIZE, c.st);
     return check(launch_reduce_frag_bf16(part, splits, batch * per, per, xu, r, (int64_t)T * r, T, r, (int)(tp / bm),
@@ -1031,7 +1057,7 @@ int big_xu(const Common& c, int stage, const void* a, int64_t lda, int64_t a_byt
   const int64_t slice = (int64_t)batch * T * r;
   int rc = big_gemm(c, stage, a, a, lda, a_bytes, u[0], u1, ldb, u_bytes, u_lin, T, r, K, batch, fn,
                     BEPI_STORE, ks, part, r, (int64_t)T * r, nullptr, true, slice, s0, s1, 0, 0, nullptr, nullptr, 1, 0,
-                    a_blk);
+                    a_blk, 0, 0, nullptr, rk.map);
   if (rc) return rc;
   StageScope fin(ST_FINALIZE, c.st);
   return check(launch_reduce_bf16(part, splits, slice, xu, slice, c.st), "split-K reduce");
@@ -1046,21 +1072,25 @@ int big_xu(const Common& c, int stage, const void* a, int64_t lda, int64_t a_byt
 // row-major h).  out_T (optional): the caller wants h as (ff, T) there; the
 // split passes' reduction writes it so, and *wrote_T says whether it did.
 int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, const void* vg, const void* vu,
-               bool v_lin, int T, int r, int ff, uint16_t* gbuf, void* out, float* part, int64_t part_cap,
+               bool v_lin, int T, int r_in, int ff, uint16_t* gbuf, void* out, float* part, int64_t part_cap,
                const float* s_vg = nullptr, const float* s_vu = nullptr, int64_t ldv = 0, int r_u = 0,
                int64_t ldv_u = 0, bool* h_blk = nullptr, void* out_T = nullptr, bool* wrote_T = nullptr) {
   const bool want_blk = h_blk && *h_blk && ff % 16 == 0;
   if (h_blk) *h_blk = false;
-  if (r_u <= 0) r_u = r;
+  if (r_u <= 0) r_u = r_in;
+  // K as XU holds it; a rank off the 32-k stages is both branches' rank
+  const Rank rk = big_rank(r_in);
+  const int r = rk.p, rows = r_in, rows_u = r_u;
+  r_u = big_rank(r_u).p;
   int fn = tune().s2fn;
   // 256 x 224 tiles (fn 7) leave most CUs idle at one or two 256-row tiles
   // of tokens; 256 x 128 tiles (fn 4) double the block count there (8B
   // layer: T=256 268 -> 245 us, T=512 298 -> 288 us; from three row tiles on
   // fn 7 is faster: T=768 349 vs 428 us).
   if (fn == 0) fn = (T <= 512 && ff % 128 == 0) ? 4 : ((ff % 224 == 0) ? 7 : 8);
-  const int64_t ldb = v_lin ? r : (ldv ? ldv : ff), ldb_u = v_lin ? r_u : (ldv_u ? ldv_u : ldb);
-  const int64_t xu_bytes = (int64_t)T * r * 2, v_bytes = (int64_t)(v_lin ? ff : r) * ldb * wbytes(c);
-  const int64_t xuu_bytes = (int64_t)T * r_u * 2, vu_bytes = (int64_t)(v_lin ? ff : r_u) * ldb_u * wbytes(c);
+  const int64_t ldb = v_lin ? rows : (ldv ? ldv : ff), ldb_u = v_lin ? rows_u : (ldv_u ? ldv_u : ldb);
+  const int64_t xu_bytes = (int64_t)T * r * 2, v_bytes = (int64_t)(v_lin ? ff : rows) * ldb * wbytes(c);
+  const int64_t xuu_bytes = (int64_t)T * r_u * 2, vu_bytes = (int64_t)(v_lin ? ff : rows_u) * ldb_u * wbytes(c);
   // 129-256 token rows on 128 x 128 K-group tiles: twice the tiles of the
   // 256-row ones, so the one-launch SwiGLU passes run without a K split (no
   // fp32 slices, no reduction), and the rows past T of a 256-row tile no
@@ -1078,7 +1108,7 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     if (want_blk) *h_blk = true;
     return big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 1, fn,
                     BEPI_GU_DUAL, std::max(r, r_u), out, ff, 0, gbuf, false, 0, s_vg, s_vu, 1, 0, nullptr, nullptr, 2,
-                    want_blk ? 1 : 0, 0, 0, 0, &du);
+                    want_blk ? 1 : 0, 0, 0, 0, &du, RankMap{}, rk.map);
   }
   // At one or two row tiles of tokens the passes split K (gu_split_plan).
   int sfn = 0, nsp = 0;
@@ -1125,7 +1155,7 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
       upart = part + (int64_t)splits * per;
       rc = big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 2, fn, BEPI_STORE,
                     ksb, part, ff, (int64_t)splits * per, nullptr, true, per, s_vg, s_vu, 0, 1, nullptr, nullptr,
-                    kg2 ? 2 : 1);
+                    kg2 ? 2 : 1, 0, 0, 0, 0, nullptr, RankMap{}, rk.map);
       if (rc) return rc;
     } else if (fused && tune().gudual && splits == splits_u && !v_lin) {
       // both passes' slices from one launch: every block its g split, then
@@ -1133,18 +1163,20 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
       const DualEntry du{r_u, xuu_bytes, r_u, ldb_u, vu_bytes, ks_u};
       rc = big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 1, fn,
                     BEPI_DUAL_F32, ks, part, ff, (int64_t)splits * per, nullptr, true, per, s_vg, s_vu, 0, 1, nullptr,
-                    nullptr, kg2 ? 2 : 1, 0, 0, 0, 0, &du);
+                    nullptr, kg2 ? 2 : 1, 0, 0, 0, 0, &du, RankMap{}, rk.map);
       if (rc) return rc;
     } else {
       rc = big_gemm(c, ST_GU_XUV_G, xu_g, nullptr, r, xu_bytes, vg, nullptr, ldb, v_bytes, v_lin, T, ff, r, 1, fn,
-                    BEPI_STORE, ks, part, ff, per, nullptr, true, per, s_vg, nullptr, 0, 1);
+                    BEPI_STORE, ks, part, ff, per, nullptr, true, per, s_vg, nullptr, 0, 1, nullptr, nullptr, 1, 0, 0, 0, 0,
+                    nullptr, RankMap{}, rk.map);
       if (rc) return rc;
       if (!fused) {
         StageScope fin(ST_FINALIZE, c.st);
         if ((rc = check(launch_reduce_bf16(part, splits, per, gbuf, per, c.st), "split-K reduce"))) return rc;
       }
       rc = big_gemm(c, ST_GU_XUV, xu_u, nullptr, r_u, xuu_bytes, vu, nullptr, ldb_u, vu_bytes, v_lin, T, ff, r_u, 1,
-                    fn, BEPI_STORE, ks_u, upart, ff, per, nullptr, true, per, s_vu, nullptr, 0, 1);
+                    fn, BEPI_STORE, ks_u, upart, ff, per, nullptr, true, per, s_vu, nullptr, 0, 1, nullptr, nullptr, 1, 0, 0, 0, 0,
+                    nullptr, RankMap{}, rk.map);
       if (rc) return rc;
     }
     StageScope fin(ST_FINALIZE, c.st);
@@ -1163,15 +1195,16 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     if (want_blk) *h_blk = true;
     return big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 1, fn,
                     BEPI_GU_DUAL, std::max(r, r_u), out, ff, 0, gbuf, false, 0, s_vg, s_vu, 1, 0, nullptr, nullptr, 1,
-                    want_blk ? 1 : 0, 0, 0, 0, &du);
+                    want_blk ? 1 : 0, 0, 0, 0, &du, RankMap{}, rk.map);
   }
   int rc = big_gemm(c, ST_GU_XUV_G, xu_g, nullptr, r, xu_bytes, vg, nullptr, ldb, v_bytes, v_lin, T, ff, r,
-                    1, fn, BEPI_STORE_FRAG, r, gbuf, ff, 0, nullptr, false, 0, s_vg);
+                    1, fn, BEPI_STORE_FRAG, r, gbuf, ff, 0, nullptr, false, 0, s_vg, nullptr, 0, 0, nullptr, nullptr, 1, 0, 0,
+                    0, 0, nullptr, RankMap{}, rk.map);
   if (rc) return rc;
   if (want_blk) *h_blk = true;
   return big_gemm(c, ST_GU_XUV, xu_u, nullptr, r_u, xuu_bytes, vu, nullptr, ldb_u, vu_bytes, v_lin, T, ff, r_u, 1,
                   fn, BEPI_SWIGLU_MEM, r_u, out, ff, 0, gbuf, false, 0, s_vu, nullptr, 1, 0, nullptr, nullptr, 1,
-                  want_blk ? 1 : 0);
+                  want_blk ? 1 : 0, 0, 0, 0, nullptr, RankMap{}, rk.map);
 }
 
 // fp8 activations for h . Ud (SVDMLP_FP8_ACT): h quantised to e4m3 per
@@ -1291,23 +1324,31 @@ int f8_down_xu(const Common& c, const uint16_t* h, const void* ud, const float* 
 }
 
 // y = XU . V with bf16 XU (T x r); bf16 y (T x dout).
-int big_v(const Common& c, const uint16_t* xu, const void* v, bool v_lin, int T, int r, int dout, char* ws,
+int big_v(const Common& c, const uint16_t* xu, const void* v, bool v_lin, int T, int r_in, int dout, char* ws,
           const Ws& L, void* y, const float* sv = nullptr, int64_t ldv = 0) {
+  const Rank rk = big_rank(r_in);
+  const int r = rk.p;
   const int fn1 = tune().s4 > 0 ? tune().s4 : 8;
-  const int64_t ldb = v_lin ? r : (ldv ? ldv : dout);
-  const int64_t xu_bytes = (int64_t)T * r * 2, v_bytes = (int64_t)(v_lin ? dout : r) * ldb * wbytes(c);
+  const int64_t ldb = v_lin ? r_in : (ldv ? ldv : dout);
+  const int64_t xu_bytes = (int64_t)T * r * 2, v_bytes = (int64_t)(v_lin ? dout : r_in) * ldb * wbytes(c);
   RankPlan pl = plan_rank(T, r, dout, fn1, 1, -1, !v_lin && c.wt == SVDMLP_BF16, ST_D_XUV);
   if (pl.kg == 1 && tune().s4 > 0 && tune().s4 != 8) pl = RankPlan{1, fn1, r, 1};
   const int fn = pl.fn, kg = pl.kg;
   const int64_t bm = kg == 2 ? 128 : 256;
-  const int ks = pl.ks;
-  const int splits = pl.splits;
+  int ks = pl.ks, splits = pl.splits;
+  if (r != r_in && splits > 1 &&  // (the slice area is sized for the ranks up to r)
+      (int64_t)splits * ((T + bm - 1) / bm * bm) * (((int64_t)dout + 32 * fn - 1) / (32 * fn) * (32 * fn)) * 4 >
+          (int64_t)(L.norm - L.part)) {
+    ks = r;
+    splits = 1;
+  }
   // the MLP block's residual add rides on the output store or the fragment-order reduction
   const uint16_t* resid = c.blk ? static_cast<const uint16_t*>(c.blk->x) : nullptr;
   if (splits == 1) {
     if (c.blk) c.blk->resid_done = true;
     return big_gemm(c, ST_D_XUV, xu, nullptr, r, xu_bytes, v, nullptr, ldb, v_bytes, v_lin, T, dout, r, 1,
-                    fn, BEPI_STORE, r, y, dout, 0, nullptr, false, 0, sv, nullptr, 0, 0, nullptr, resid, kg);
+                    fn, BEPI_STORE, r, y, dout, 0, nullptr, false, 0, sv, nullptr, 0, 0, nullptr, resid, kg, 0, 0, 0, 0, nullptr, RankMap{},
+                    rk.map);
   }
   float* part = reinterpret_cast<float*>(ws + L.part);
   const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, v_lin);
@@ -1315,7 +1356,8 @@ int big_v(const Common& c, const uint16_t* xu, const void* v, bool v_lin, int T,
     if (c.blk) c.blk->resid_done = true;
     const int64_t tp = (T + bm - 1) / bm * bm, np = ((int64_t)dout + 32 * fn - 1) / (32 * fn) * (32 * fn), per = tp * np;
     int rc = big_gemm(c, ST_D_XUV, xu, nullptr, r, xu_bytes, v, nullptr, ldb, v_bytes, v_lin, T, dout, r, 1, fn,
-                      BEPI_STORE, ks, part, dout, per, nullptr, true, per, sv, nullptr, 0, 1, nullptr, nullptr, kg);
+                      BEPI_STORE, ks, part, dout, per, nullptr, true, per, sv, nullptr, 0, 1, nullptr, nullptr, kg, 0, 0, 0, 0,
+                      nullptr, RankMap{}, rk.map);
     if (rc) return rc;
     StageScope fin(ST_FINALIZE, c.st);
     return check(launch_reduce_frag_bf16(part, splits, per, per, static_cast<uint16_t*>(y), dout, (int64_t)T * dout,
@@ -1325,7 +1367,8 @@ int big_v(const Common& c, const uint16_t* xu, const void* v, bool v_lin, int T,
   }
   const int64_t slice = (int64_t)T * dout;
   int rc = big_gemm(c, ST_D_XUV, xu, nullptr, r, xu_bytes, v, nullptr, ldb, v_bytes, v_lin, T, dout, r,
-                    1, fn, BEPI_STORE, ks, part, dout, 0, nullptr, true, slice, sv);
+                    1, fn, BEPI_STORE, ks, part, dout, 0, nullptr, true, slice, sv, nullptr, 0, 0, nullptr, nullptr, 1, 0, 0,
+                    0, 0, nullptr, RankMap{}, rk.map);
   if (rc) return rc;
   StageScope fin(ST_FINALIZE, c.st);
   return check(launch_reduce_bf16(part, splits, slice, static_cast<uint16_t*>(y), slice, c.st), "split-K reduce");
@@ -2026,7 +2069,7 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
     return check(launch_transpose_bf16(hn, ff, static_cast<uint16_t*>(h), T, (int)T, (int)ff, c.st), "h transpose");
   }
 
-  if (big_ok(c, vec, {T * d * 2, d * r * 2, r * ff * 2, T * ff * 2}, {d, r})) {
+  if (big_ok(c, vec, {T * d * 2, d * r * 2, r * ff * 2, T * ff * 2}, {d}) && big_rank_ok(c, r)) {
     const void* us[2] = {ug, uu};
     const float* sus[2] = {s_ug, s_uu};
     if ((rc = big_xu(c, ST_GU_XU, x, d, T * d * 2, us, u_lin, T, d, r, 2, ws, L, fp8 ? sus : nullptr))) return rc;
@@ -2038,7 +2081,7 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
     // pass into the caller's buffer
     uint16_t* hn = out_t ? reinterpret_cast<uint16_t*>(ws + L.h) : static_cast<uint16_t*>(h);
     bool wrote_T = false;
-    if ((rc = big_swiglu(c, xu, xu + T * r, vg, vu, v_lin, T, r, ff, gbuf, hn, reinterpret_cast<float*>(ws + L.part),
+    if ((rc = big_swiglu(c, xu, xu + T * big_rank(r).p, vg, vu, v_lin, T, r, ff, gbuf, hn, reinterpret_cast<float*>(ws + L.part),
                          (int64_t)(L.norm - L.part), fp8 ? s_vg : nullptr, fp8 ? s_vu : nullptr, 0, 0, 0, nullptr,
                          out_t ? h : nullptr, &wrote_T)) ||
         !out_t || wrote_T)
@@ -2111,7 +2154,7 @@ int svdmlp_xuv(const void* x, const void* u, const void* v, const float* s_u, co
                         "decode XU.V");
   }
 
-  if (!x_t && big_ok(c, vec, {T * din * 2, din * r * 2, r * dout * 2, T * dout * 2}, {din, r})) {
+  if (!x_t && big_ok(c, vec, {T * din * 2, din * r * 2, r * dout * 2, T * dout * 2}, {din}) && big_rank_ok(c, r)) {
     const void* us[1] = {u};
     const float* sus[1] = {s_u};
     if ((rc = big_xu(c, ST_D_XU, x, din, T * din * 2, us, u_lin, T, din, r, 1, ws, L, fp8 ? sus : nullptr)))
@@ -2301,7 +2344,8 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
   if (mfma_layer)
     return decode_layer(c, x, ug, vg, uu, vu, ud, vd, y, T, d, ff, r_gu, r_d, ws, L, ld);
   const bool big = big_ok(c, vec, {T * d * 2, d * ld.u * 2, r_gu * ld.v * 2, T * ff * 2, ff * ld.ud * 2, r_d * ld.vd * 2},
-                          {d, r_gu, ff, r_d});
+                          {d, ff}) &&
+                   (ld.dense ? big_rank_ok(c, r_gu) && big_rank_ok(c, r_d) : r_gu % 32 == 0 && r_d % 32 == 0);
   if (!ld.dense && (T <= kDecodeMaxT || !big))
     return fail("factors with padded rows: no kernel takes this shape (the decode layers need d, ranks and ff in "
                 "multiples of 128, 128 and 64, the large-tile path more than %lld tokens)", (long long)kDecodeMaxT);
@@ -2346,9 +2390,9 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
     const uint16_t* xu = reinterpret_cast<const uint16_t*>(ws + L.xu_bf16);
     uint16_t* hbuf = reinterpret_cast<uint16_t*>(ws + L.h);
     uint16_t* gbuf = reinterpret_cast<uint16_t*>(ws + L.g);
-    const bool f8a = fp8_act && f8_down_ok(T, ff, r_d, ld.ud);
+    const bool f8a = fp8_act && r_d % 32 == 0 && f8_down_ok(T, ff, r_d, ld.ud);
     bool hblk = !f8a && tune().hblk;
-    if ((rc = big_swiglu(c, xu, xu + T * r_gu, vg, vu, v_lin, T, r_gu, ff, gbuf, hbuf,
+    if ((rc = big_swiglu(c, xu, xu + T * big_rank(r_gu).p, vg, vu, v_lin, T, r_gu, ff, gbuf, hbuf,
                          reinterpret_cast<float*>(ws + L.part), (int64_t)(L.norm - L.part), S[1], S[3], ld.v, 0, 0,
                          &hblk)))
       return rc;

@@ -8,8 +8,15 @@ namespace {
 
 template <int FN, bool BK, int EPI, bool F32 = false, bool F8 = false, int NW = 8, int NS = 4, int KG = 1, bool TR = false>
 hipError_t go(const BigParams& p, int splits, int batch, hipStream_t st) {
-  using C = BigCfg<FN, BK, EPI, F32, F8, NW, NS, KG, TR>;
   dim3 grid(p.tiles > 0 ? p.tiles : p.mtiles * p.ntiles, splits, batch);
+  using C = BigCfg<FN, BK, EPI, F32, F8, NW, NS, KG, TR>;
+  if (!C::RM && (p.nmap[0].shift || p.kmap[0].shift)) {  // fp8 B: instances of their own, 8 waves
+    if constexpr (F8 && NW == 8) {
+      hipLaunchKernelGGL(big_gemm_kernel<BigCfgRM<C>>, grid, dim3(C::THREADS), 0, st, p);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
   hipLaunchKernelGGL(big_gemm_kernel<C>, grid, dim3(C::THREADS), 0, st, p);
   return hipGetLastError();
 }

@@ -193,6 +193,10 @@ enum BigEpi : int {
   BEPI_DUAL_F32 = 5
 };
 
+struct RankMap {
+  int cut = 0x7fffffff, shift = 0;
+};
+
 struct BigParams {
   const void* a[2];  // per batch entry
   const void* b[2];
@@ -229,6 +233,14 @@ struct BigParams {
   // split, its fragment-order outputs compact from tile0; 0: all mtiles x ntiles
   int tile0, tiles;
   int k_split;
+  // Ranks off the 32-k stages (RankMap): the rank-r intermediate XU is held
+  // r rounded up to 64 columns wide, its columns from `cut` (the last whole
+  // multiple of 64) on moved up by `shift`, zeros in between.  nmap: the X.U
+  // product writes it so (output column n >= cut takes B column n - shift,
+  // the gap none); kmap: the product that reads it (B rows of stages from cut
+  // on lie `shift` rows earlier: the last 64 rows of V, of which the first
+  // `shift` meet the zeros).  No B row or column outside the matrix is read.
+  RankMap nmap[2], kmap[2];
 };
 
 template <int FN_, bool B_KC_, int EPI_, bool OUT_F32_, bool FP8_B_ = false, int NW_ = 8, int NS_ = 4, int KG_ = 1,
@@ -250,6 +262,10 @@ struct BigCfg {
   // instance: its block-to-tile arithmetic, compiled into every instance,
   // cost the fp8-B ones ~20 VGPRs and the 256 x 256 fp8-B ones a spill.
   static constexpr bool TR = TR_;
+  // RM: the launch may carry rank maps (BigParams::nmap, kmap).  The fp8
+  // instances have it apart (BigCfgRM): in their loop it cost the 70B layer
+  // 0.5% (the bf16 ones measure the same with and without).
+  static constexpr bool RM = !FP8_B_;
   static constexpr int WT = NW / KG;                 // wave tiles per block
   static constexpr int THREADS = 64 * NW;
   static constexpr int BM = KG == 2 ? 128 : 256;
@@ -283,6 +299,11 @@ struct BigCfg {
   static_assert(STAGES >= 3 && STAGES * STAGE <= 160 * 1024, "LDS budget");
   // K groups add their sums through LDS: half of each wave's fragments
   static_assert(KG == 1 || NW * (FM / 2) * FN * 1024 <= STAGES * STAGE, "K-group exchange fits the stages' LDS");
+};
+
+template <class C>
+struct BigCfgRM : C {
+  static constexpr bool RM = true;
 };
 
 template <class C>
@@ -371,6 +392,10 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         a_voff[i] = row < p.M ? (uint32_t)row * lda2 + (uint32_t)(a_kk * 2) : kOOB;
       }
     }
+    // output column n's column in B, and whether it has one (RankMap)
+    const RankMap nm = p.nmap[zb], km = p.kmap[zb];
+    auto b_col = [&](int n) { return C::RM && n >= nm.cut ? n - nm.shift : n; };
+    auto b_has = [&](int n) { return n < N && (!C::RM || n < nm.cut || n >= nm.cut + nm.shift); };
     // B natural: instruction i fills LDS k-row 2*(wave + NW*i) + lane/32, slot
     // lane%32 -> logical column 16*((slot/2) ^ swz(row)) + 8*(slot%2).
     // B Linear: like A with rows n.
@@ -381,7 +406,7 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
 #pragma unroll
       for (int i = 0; i < C::B_UNITS; ++i) {
         const int row = row0 + 16 * NW * i;
-        b_voff[i] = (row < BN && n0 + row < N) ? (uint32_t)(n0 + row) * ldb2 + (uint32_t)(kk * 2) : kOOB;
+        b_voff[i] = (row < BN && b_has(n0 + row)) ? (uint32_t)b_col(n0 + row) * ldb2 + (uint32_t)(kk * 2) : kOOB;
       }
     } else if constexpr (C::FP8_B) {
       // fp8 natural: instruction i fills k-rows 4*(wave + NW*i) + lane/16
@@ -391,7 +416,7 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
       for (int i = 0; i < C::B_UNITS; ++i) {
         const int kk = 4 * (wave + NW * i) + (lane >> 4);
         const int col = 16 * ((lane & 15) ^ f8nat_swz(kk));
-        b_voff[i] = (col < BN && n0 + col < N) ? (uint32_t)kk * (uint32_t)ldb + (uint32_t)(n0 + col) : kOOB;
+        b_voff[i] = (col < BN && b_has(n0 + col)) ? (uint32_t)kk * (uint32_t)ldb + (uint32_t)b_col(n0 + col) : kOOB;
       }
     } else if constexpr (C::B_PITCH == 384) {
       // 384-byte rows: instruction i fills bytes (wave + NW*i) KB .. +1 KB of
@@ -402,7 +427,7 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         const int pos = (wave + NW * i) * 1024 + 16 * lane;
         const int kk = pos / 384, byte = pos % 384;
         const int col = 16 * ((byte >> 5) ^ b384_swz(kk)) + 8 * ((byte >> 4) & 1);
-        b_voff[i] = n0 + col < N ? (uint32_t)kk * ldb2 + (uint32_t)((n0 + col) * 2) : kOOB;
+        b_voff[i] = b_has(n0 + col) ? (uint32_t)kk * ldb2 + (uint32_t)(b_col(n0 + col) * 2) : kOOB;
       }
     } else {
       // instruction i fills RPI k-rows from RPI * (wave + NW * i), LPR lanes per
@@ -415,7 +440,7 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
       for (int i = 0; i < C::B_UNITS; ++i) {
         const int kk = RPI * (wave + NW * i) + lane / LPR;
         const int col = 16 * ((q >> 1) ^ bnat_swz(kk)) + 8 * (q & 1);
-        b_voff[i] = (col < BN && n0 + col < N) ? (uint32_t)kk * ldb2 + (uint32_t)((n0 + col) * 2) : kOOB;
+        b_voff[i] = (col < BN && b_has(n0 + col)) ? (uint32_t)kk * ldb2 + (uint32_t)(b_col(n0 + col) * 2) : kOOB;
       }
     }
 
@@ -430,7 +455,8 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         dma16(live ? ra : r_none, a_voff[d], ((uint32_t)k0 << kshift) + ksub, lbase + s * C::A_BYTES + (wave + NW * d) * 1024);
       } else {
         const int i = d - C::A_UNITS;
-        const uint32_t soff = C::B_KC ? (uint32_t)k0 * 2u : (C::FP8_B ? (uint32_t)k0 * (uint32_t)ldb : (uint32_t)k0 * ldb2);
+        const uint32_t kr = (uint32_t)(C::RM && k0 >= km.cut ? k0 - km.shift : k0);
+        const uint32_t soff = C::B_KC ? kr * 2u : (C::FP8_B ? kr * (uint32_t)ldb : kr * ldb2);
         dma16(live ? rb : r_none, b_voff[i], soff, lbase + B_REGION + s * C::B_BYTES + (wave + NW * i) * 1024);
       }
     };
@@ -644,7 +670,8 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         if (!FRAG && !ffrag && n >= N) continue;  // N % 8 == 0: n < N implies n + 3 < N
         f32x4 v = acc[i][j];
         if constexpr (C::FP8_B)
-          if (n < N) v *= *reinterpret_cast<const f32x4*>(p.scale[zb] + n);  // per-column dequant
+          // per-column dequant (fp8 ranks keep the map's bounds at multiples of 16: the column's is a scalar)
+          if (n < N) v *= *reinterpret_cast<const f32x4*>(p.scale[zb] + (C::RM ? b_col(n0 + wn0 + 16 * j) + 4 * lg : n));
         const int64_t fo = frag0 + (int64_t)(i * FN + j) * 256;
         if constexpr (FRAG) {
           // (a dual block's gate values go to gmem, its own buffer)

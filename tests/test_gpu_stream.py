@@ -190,3 +190,29 @@ def test_decode_layer_phase2_splits(gpu, d, ff, ranks, T):
         assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
     (ws,) = ops._WS_CACHE.values()
     assert not any(ws[2560:4096].view(torch.int32).cpu().tolist()) and not ops.workspace_status()
+
+
+# Large-tile path with ranks off the 32-k stages (XU held in whole 64-column
+# blocks, the last one the last 64 ranks with zeros for those it repeats): one
+# rank piece past a block (72), one short of it (504 = 7 * 64 + 56), in and off
+# the 16 columns of an fp8 piece, equal and different down ranks; token counts
+# of every plan (split passes, K-group tiles, one launch of both passes).
+@pytest.mark.parametrize("T", [65, 128, 200, 300, 520, 1030])
+@pytest.mark.parametrize("kind", ["natural", "linear", "fp8"])
+@pytest.mark.parametrize("shape", [inputs.LayerShape(1024, 2048, 336, 504), inputs.LayerShape(256, 1792, 72, 1160),
+                                   inputs.LayerShape(512, 4096, 496, 80)])
+def test_ranks_off_the_stages(gpu, shape, kind, T):
+    xb, wide, xt, ft = _layer(shape, T, 700 + T, kind, gpu)
+    h = ops.fused_gate_up(xt, *ft[:4])
+    assert _rel(_np(h), O.fused_gate_up_ref(xb, *wide[:4], dtype="bfloat16")) < TOL
+    y = ops.fused_xuv(h, *ft[4:])
+    assert _rel(_np(y), O.fused_xuv_ref(_np(h), *wide[4:], dtype="bfloat16")) < TOL
+    out = ops.svd_mlp(xt, *ft)
+    assert _rel(_np(out), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+    if kind != "fp8" or shape.rd % 16 == 0:  # (the general kernel, which sums K splits by float atomics, has the others)
+        assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
+    if kind == "natural":
+        gain = torch.rand(shape.d, device=gpu) + 0.5
+        blk = ops.svd_mlp_block(xt, gain, *ft)
+        xn = (xt.float() * torch.rsqrt(xt.float().pow(2).mean(1, keepdim=True) + 1e-5) * gain).bfloat16()
+        assert _rel(_np(blk), _np((xt.float() + ops.svd_mlp(xn, *ft).float()).bfloat16())) < TOL
