@@ -1094,16 +1094,42 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
   // 129-256 token rows on 128 x 128 K-group tiles: twice the tiles of the
   // 256-row ones, so the one-launch SwiGLU passes run without a K split (no
   // fp32 slices, no reduction), and the rows past T of a 256-row tile no
-  // longer cost MFMAs.  Faster on every shape measured, also where the tiles
-  // fill half the CUs (layer, two alternating runs, 256-row split passes ->
-  // these: 8B T=160 / 200 / 256 154.2 / 161.9 / 169.7 -> 135.5 / 143.1 /
-  // 155.6 us; 3B (3072, 8192, 1792) T=160 / 256 104.6 / 109.2 -> 98.5 / 108.0;
-  // (1024, 4096, 512) 66.5 / 62.8 -> 58.8 / 55.5).  Up to 512 rows while the
-  // tiles fit one round of the CUs (3B T=384 / 512: 128.1 / 145.0 -> 116.1 /
-  // 124.7 us; the 8B shape's 336 tiles at T=384 would take two rounds).
+  // longer cost MFMAs (8B layer, 256-row split passes -> these: T=160 / 200
+  // 149 / 155 -> 140 / 147 us, T=256 160 either way; (1024, 4096, 512) T=256
+  // 58 -> 52).  Up to 512 rows while the tiles fit one round of the CUs (3B
+  // (3072, 8192, 1792) T=384 / 512: 126 / 131 -> 114 / 123 us; the 8B shape's
+  // 336 tiles at T=384 would take two rounds).
   const int64_t kg_tiles = (int64_t)(T + 127) / 128 * ((ff + 127) / 128);
   if (tune().gukgu && T > 128 && (tune().gukgu >= 2 ? kg_tiles <= tune().split : T <= 256) && fn == 4 &&
       c.wt == SVDMLP_BF16 && !v_lin && tune().gudual && r % 64 == 0 && r_u % 64 == 0 && ff % 128 == 0) {
+    // At most half a round of tiles: half the CUs would run both branches in
+    // turn while the rest idle, so the branches go side by side as batch
+    // entries, in K splits that fill the CUs, and one reduction applies
+    // SiLU(g) (as the split passes below).  Splits of 512 k or more: at 256 k
+    // the fill of each block's pipeline and the slices cost what the CUs gain
+    // ((4096, 1792, 1024) T=256 67.8 us, (1024, 3584, 256) 56).  us, both
+    // branches in a block -> a branch a block: 3B T=130 / 200 / 256 95.3 /
+    // 101.7 / 107.4 -> 89.8 / 92.2 / 94.8, (2560, 6912, 1408) T=256 85.0 ->
+    // 76.6, (4096, 1792, 1024) T=130 / 256 72.0 / 67.0 -> 67.3 / 62.0,
+    // (2048, 5632, 1152) T=256 69.8 -> 66.3.
+    const int64_t per2 = (int64_t)((T + 127) / 128 * 128) * ff;
+    int64_t sp = std::min({(int64_t)4, tune().split / (2 * kg_tiles), (int64_t)(r / 512), part_cap / (2 * per2 * 4)});
+    if (sp >= 1 && tune().gupair && r == r_u && ldb == ldb_u) {
+      const int ksb = (int)(((r + sp - 1) / sp + 63) / 64 * 64);
+      sp = (r + ksb - 1) / ksb;
+      const int rc = big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 2, 4,
+                              BEPI_STORE, ksb, part, ff, sp * per2, nullptr, true, per2, s_vg, s_vu, 0, 1, nullptr,
+                              nullptr, 2, 0, 0, 0, 0, nullptr, RankMap{}, rk.map);
+      if (rc) return rc;
+      StageScope fin(ST_FINALIZE, c.st);
+      const bool tr = out_T && T % 8 == 0;
+      if (wrote_T) *wrote_T = tr;
+      return check(launch_reduce_frag_bf16(part + sp * per2, (int)sp, per2, per2,
+                                           static_cast<uint16_t*>(tr ? out_T : out), tr ? T : ff, (int64_t)T * ff, T, ff,
+                                           (T + 127) / 128, ff / 128, 4, 8, 1, c.st, nullptr, nullptr, 2, part, (int)sp,
+                                           tr),
+                   "split-K SwiGLU reduce");
+    }
     const DualEntry du{r_u, xuu_bytes, r_u, ldb_u, vu_bytes};
     if (want_blk) *h_blk = true;
     return big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 1, fn,

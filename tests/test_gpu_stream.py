@@ -216,3 +216,19 @@ def test_ranks_off_the_stages(gpu, shape, kind, T):
         blk = ops.svd_mlp_block(xt, gain, *ft)
         xn = (xt.float() * torch.rsqrt(xt.float().pow(2).mean(1, keepdim=True) + 1e-5) * gain).bfloat16()
         assert _rel(_np(blk), _np((xt.float() + ops.svd_mlp(xn, *ft).float()).bfloat16())) < TOL
+
+
+# 129-256 tokens where the 128 x 128 K-group tiles fill at most half the CUs:
+# the branches as batch entries in 1, 2 and 4 K splits (the last one ragged at
+# rank 1088 and 2112), ragged last row tiles, the transposed result, a rank at
+# the line (512) and one below it (448: both branches in a block).
+@pytest.mark.parametrize("T", [129, 200, 256])
+@pytest.mark.parametrize("ff,r", [(1792, 1088), (1792, 2112), (8192, 512), (8192, 448), (128, 2048)])
+def test_gate_up_paired_kgroup_tiles(gpu, ff, r, T):
+    xb, wide, xt, ft = _layer(inputs.LayerShape(512, ff, r, 128), T, T + r, "natural", gpu)
+    h = ops.fused_gate_up(xt, *ft[:4])
+    assert _rel(_np(h), O.fused_gate_up_ref(xb, *wide[:4], dtype="bfloat16")) < TOL
+    assert torch.equal(ops.fused_gate_up(xt, *ft[:4]).view(torch.int16), h.view(torch.int16))
+    if T % 8 == 0:
+        assert torch.equal(ops.fused_gate_up(xt, *ft[:4], out_transposed=True).t(), h)
+    assert _rel(_np(ops.svd_mlp(xt, *ft)), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
