@@ -654,8 +654,10 @@ int big_gemm(const Common& c, int stage, const void* a0, const void* a1, int64_t
              bool out_f32 = false, int64_t out_sstride = 0, const float* s0 = nullptr, const float* s1 = nullptr,
              int gfrag = 0, int out_frag = 0, const Entry1* e1 = nullptr, const uint16_t* resid = nullptr,
              int kg = 1, int out_blk = 0, int a_blk = 0, int tile0 = 0, int tiles = 0,
-             const DualEntry* du = nullptr, const RankMap& nmap = RankMap{}, const RankMap& kmap = RankMap{}) {
+             const DualEntry* du = nullptr, const RankMap& nmap = RankMap{}, const RankMap& kmap = RankMap{},
+             uint16_t* glo = nullptr) {
   BigParams p{};
+  p.glo = glo;
   p.nmap[0] = p.nmap[1] = nmap;  // ranks off the stages are the same for both entries
   p.kmap[0] = p.kmap[1] = kmap;
   p.tile0 = tile0;
@@ -1075,6 +1077,10 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
                bool v_lin, int T, int r_in, int ff, uint16_t* gbuf, void* out, float* part, int64_t part_cap,
                const float* s_vg = nullptr, const float* s_vu = nullptr, int64_t ldv = 0, int r_u = 0,
                int64_t ldv_u = 0, bool* h_blk = nullptr, void* out_T = nullptr, bool* wrote_T = nullptr) {
+  // Ranks off the stages and transposed results at token counts off 8 keep g
+  // in 32 bits up to SiLU (as the split passes' slices do).
+  const bool g32 = big_rank(r_in).map.shift || (out_T && T % 8);
+  uint16_t* const glo = g32 ? static_cast<uint16_t*>(out) : nullptr;
   const bool want_blk = h_blk && *h_blk && ff % 16 == 0;
   if (h_blk) *h_blk = false;
   if (r_u <= 0) r_u = r_in;
@@ -1134,7 +1140,7 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     if (want_blk) *h_blk = true;
     return big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 1, fn,
                     BEPI_GU_DUAL, std::max(r, r_u), out, ff, 0, gbuf, false, 0, s_vg, s_vu, 1, 0, nullptr, nullptr, 2,
-                    want_blk ? 1 : 0, 0, 0, 0, &du, RankMap{}, rk.map);
+                    want_blk ? 1 : 0, 0, 0, 0, &du, RankMap{}, rk.map, glo);
   }
   // At one or two row tiles of tokens the passes split K (gu_split_plan).
   int sfn = 0, nsp = 0;
@@ -1159,13 +1165,13 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
   }
   if (!kg2) per = (int64_t)((T + 255) / 256 * 256) * np;
   const int bm = kg2 ? 128 : 256;
-  if (nsp >= 2 && fn == 4 && r >= 32 * nsp && r_u >= 32 * nsp && nsp * per * 4 <= part_cap) {
+  if (nsp >= 2 && fn == 4 && r >= 32 * nsp && r_u >= 32 * nsp && (g32 ? 2 : 1) * nsp * per * 4 <= part_cap) {
     fn = sfn;
     // Both passes' slices side by side when the area holds them: one
-    // reduction then rounds g from its slices and applies SiLU(g) to the u
-    // sum (bitwise the two-reduction result, one launch and the bf16 g round
-    // trip fewer); else g is reduced to bf16 before the u pass reuses the area.
-    const bool fused = tune().gufuse && (int64_t)(splits + splits_u) * per * 4 <= part_cap;
+    // reduction then sums g and applies SiLU(g) to the u sum (one launch and
+    // the bf16 g round trip fewer); else g is reduced to bf16 before the u pass
+    // reuses the area.
+    const bool fused = (tune().gufuse || g32) && (int64_t)(splits + splits_u) * per * 4 <= part_cap;
     float* upart = fused ? part + (int64_t)splits * per : part;
     int rc;
     // An even number of splits as half as many per branch, the branches side
@@ -1221,16 +1227,16 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     if (want_blk) *h_blk = true;
     return big_gemm(c, ST_GU_XUV_DUAL, xu_g, xu_u, r, xu_bytes, vg, vu, ldb, v_bytes, v_lin, T, ff, r, 1, fn,
                     BEPI_GU_DUAL, std::max(r, r_u), out, ff, 0, gbuf, false, 0, s_vg, s_vu, 1, 0, nullptr, nullptr, 1,
-                    want_blk ? 1 : 0, 0, 0, 0, &du, RankMap{}, rk.map);
+                    want_blk ? 1 : 0, 0, 0, 0, &du, RankMap{}, rk.map, glo);
   }
   int rc = big_gemm(c, ST_GU_XUV_G, xu_g, nullptr, r, xu_bytes, vg, nullptr, ldb, v_bytes, v_lin, T, ff, r,
-                    1, fn, BEPI_STORE_FRAG, r, gbuf, ff, 0, nullptr, false, 0, s_vg, nullptr, 0, 0, nullptr, nullptr, 1, 0, 0,
-                    0, 0, nullptr, RankMap{}, rk.map);
+                    1, fn, BEPI_STORE_FRAG, r, gbuf, ff, 0, nullptr, false, 0, s_vg, nullptr, 0, 0, nullptr, nullptr, 1,
+                    want_blk && glo ? 1 : 0, 0, 0, 0, nullptr, RankMap{}, rk.map, glo);
   if (rc) return rc;
   if (want_blk) *h_blk = true;
   return big_gemm(c, ST_GU_XUV, xu_u, nullptr, r_u, xuu_bytes, vu, nullptr, ldb_u, vu_bytes, v_lin, T, ff, r_u, 1,
                   fn, BEPI_SWIGLU_MEM, r_u, out, ff, 0, gbuf, false, 0, s_vu, nullptr, 1, 0, nullptr, nullptr, 1,
-                  want_blk ? 1 : 0, 0, 0, 0, nullptr, RankMap{}, rk.map);
+                  want_blk ? 1 : 0, 0, 0, 0, nullptr, RankMap{}, rk.map, glo);
 }
 
 // fp8 activations for h . Ud (SVDMLP_FP8_ACT): h quantised to e4m3 per

@@ -10,6 +10,13 @@ template <int FN, bool BK, int EPI, bool F32 = false, bool F8 = false, int NW = 
 hipError_t go(const BigParams& p, int splits, int batch, hipStream_t st) {
   dim3 grid(p.tiles > 0 ? p.tiles : p.mtiles * p.ntiles, splits, batch);
   using C = BigCfg<FN, BK, EPI, F32, F8, NW, NS, KG, TR>;
+  if (p.glo) {
+    if constexpr (NW == 8 && (EPI == BEPI_STORE_FRAG || EPI == BEPI_SWIGLU_MEM || EPI == BEPI_GU_DUAL)) {
+      hipLaunchKernelGGL(big_gemm_kernel<BigCfgG32<C>>, grid, dim3(C::THREADS), 0, st, p);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
   if (!C::RM && (p.nmap[0].shift || p.kmap[0].shift)) {  // fp8 B: instances of their own, 8 waves
     if constexpr (F8 && NW == 8) {
       hipLaunchKernelGGL(big_gemm_kernel<BigCfgRM<C>>, grid, dim3(C::THREADS), 0, st, p);
@@ -125,17 +132,16 @@ __global__ __launch_bounds__(256) void reduce_frag_bf16_kernel(const float* in, 
 #pragma unroll
     for (int k = 0; k < PER; ++k) a[k] += b[k];
   }
-  if (gsl) {  // SwiGLU with the gate as fp32 slices: g = bf16(sum in split order), then out = SiLU(g) * sum
+  if (gsl) {  // SwiGLU with the gate as fp32 slices, summed in split order: out = SiLU(g) * sum
     const float* gp = gsl + (int64_t)zb * bstride + (int64_t)unit * Q * 4 + 4 * threadIdx.x;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       f32x4 g = *reinterpret_cast<const f32x4*>(gp + 1024 * k);
       for (int s = 1; s < gsplits; ++s) g += *reinterpret_cast<const f32x4*>(gp + s * sstride + 1024 * k);
-      const uint32_t g01 = pack_bf16x2(g.x, g.y), g23 = pack_bf16x2(g.z, g.w);
-      a[k].x *= silu_f32(bf16_bits_to_f32(g01 & 0xffffu));
-      a[k].y *= silu_f32(bf16_bits_to_f32(g01 >> 16));
-      a[k].z *= silu_f32(bf16_bits_to_f32(g23 & 0xffffu));
-      a[k].w *= silu_f32(bf16_bits_to_f32(g23 >> 16));
+      a[k].x *= silu_f32(g.x);
+      a[k].y *= silu_f32(g.y);
+      a[k].z *= silu_f32(g.z);
+      a[k].w *= silu_f32(g.w);
     }
   } else if (gate) {  // SwiGLU: out = SiLU(g) * sum, g bf16 in the same fragment order
     const uint16_t* gp = gate + (int64_t)zb * bstride + (int64_t)unit * Q * 4 + 4 * threadIdx.x;

@@ -241,6 +241,10 @@ struct BigParams {
   // on lie `shift` rows earlier: the last 64 rows of V, of which the first
   // `shift` meet the zeros).  No B row or column outside the matrix is read.
   RankMap nmap[2], kmap[2];
+  // Gate values in 32 bits (G32 instances; null: bf16): gmem then holds their
+  // upper halves and glo, the h buffer itself, their lower ones, each lane's
+  // where its own h values go.
+  uint16_t* glo;
 };
 
 template <int FN_, bool B_KC_, int EPI_, bool OUT_F32_, bool FP8_B_ = false, int NW_ = 8, int NS_ = 4, int KG_ = 1,
@@ -266,6 +270,7 @@ struct BigCfg {
   // instances have it apart (BigCfgRM): in their loop it cost the 70B layer
   // 0.5% (the bf16 ones measure the same with and without).
   static constexpr bool RM = !FP8_B_;
+  static constexpr bool G32 = false;  // gate values in 32 bits between the passes (BigCfgG32)
   static constexpr int WT = NW / KG;                 // wave tiles per block
   static constexpr int THREADS = 64 * NW;
   static constexpr int BM = KG == 2 ? 128 : 256;
@@ -304,6 +309,17 @@ struct BigCfg {
 template <class C>
 struct BigCfgRM : C {
   static constexpr bool RM = true;
+};
+
+// Gate values carried between the passes in all 32 bits, for the calls whose
+// SwiGLU the 128 x 128 kernel would take with g in its accumulators (ranks off
+// the stages, transposed results at token counts off 8): 16 more bits a value
+// written and read back by the lane that needs them, no buffer more.
+// 8B layer at rank 2744, T=512 / 1024, g in bf16 -> in 32 bits: 214 / 314 ->
+// 217 / 330 us (the 128 x 128 kernel: 946 / 1578).
+template <class C>
+struct BigCfgG32 : C {
+  static constexpr bool RM = true, G32 = true;
 };
 
 template <class C>
@@ -664,6 +680,19 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
       if (C::KG == 2 && (i / (FM / 2)) != kg) continue;  // the partner wave's rows
       const int m = m0 + wm0 + 16 * i + lr;
       if (!FRAG && !ffrag && m >= p.M) continue;
+      // element offset of this lane's h values in the row's fragment j
+      const auto h_off = [&](int n) {
+        return p.out_blk ? (((int64_t)(m >> 4) * (N >> 4) + (n >> 4)) * 256 + (m & 15) * 16 + (n & 15))
+                         : (int64_t)m * ldo + n;
+      };
+      u32x2 gl[C::G32 && EP == BEPI_SWIGLU_MEM ? FN : 1];  // this lane's own stores of the g pass; a row at a time
+      if constexpr (C::G32 && EP == BEPI_SWIGLU_MEM) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const int n = n0 + wn0 + 16 * j + 4 * lg;
+          gl[j] = *reinterpret_cast<const u32x2*>(p.glo + (n < N ? h_off(n) : 0));
+        }
+      }
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         const int n = n0 + wn0 + 16 * j + 4 * lg;
@@ -676,6 +705,15 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         if constexpr (FRAG) {
           // (a dual block's gate values go to gmem, its own buffer)
           uint16_t* const fout = C::EPI == BEPI_GU_DUAL ? const_cast<uint16_t*>(p.gmem) : reinterpret_cast<uint16_t*>(p.out);
+          if constexpr (C::G32) {
+            const u32x4 b = __builtin_bit_cast(u32x4, v);
+            *reinterpret_cast<u32x2*>(fout + fo) =
+                u32x2{(b.x >> 16) | (b.y & 0xffff0000u), (b.z >> 16) | (b.w & 0xffff0000u)};
+            if (m < p.M && n < N)
+              *reinterpret_cast<u32x2*>(p.glo + h_off(n)) =
+                  u32x2{(b.x & 0xffffu) | (b.y << 16), (b.z & 0xffffu) | (b.w << 16)};
+            continue;
+          }
           *reinterpret_cast<u32x2*>(fout + fo) = u32x2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
           continue;
         }
@@ -690,10 +728,16 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
           *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(outp) + (ffrag ? fo : o)) = v;
         } else if constexpr (EP == BEPI_SWIGLU_MEM) {
           const u32x2 g = gv[i][j];
-          const float g0 = bf16_bits_to_f32(g.x & 0xffffu), g1 = bf16_bits_to_f32(g.x >> 16);
-          const float g2 = bf16_bits_to_f32(g.y & 0xffffu), g3 = bf16_bits_to_f32(g.y >> 16);
-          const int64_t ob = p.out_blk ? (((int64_t)(m >> 4) * (N >> 4) + (n >> 4)) * 256 + (m & 15) * 16 + (n & 15)) : o;
-          *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(outp) + ob) =
+          float g0 = bf16_bits_to_f32(g.x & 0xffffu), g1 = bf16_bits_to_f32(g.x >> 16);
+          float g2 = bf16_bits_to_f32(g.y & 0xffffu), g3 = bf16_bits_to_f32(g.y >> 16);
+          if constexpr (C::G32) {
+            const u32x2 l = gl[j];
+            g0 = __builtin_bit_cast(float, (g.x << 16) | (l.x & 0xffffu));
+            g1 = __builtin_bit_cast(float, (g.x & 0xffff0000u) | (l.x >> 16));
+            g2 = __builtin_bit_cast(float, (g.y << 16) | (l.y & 0xffffu));
+            g3 = __builtin_bit_cast(float, (g.y & 0xffff0000u) | (l.y >> 16));
+          }
+          *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(outp) + h_off(n)) =
               u32x2{pack_bf16x2(silu_f32(g0) * v.x, silu_f32(g1) * v.y),
                     pack_bf16x2(silu_f32(g2) * v.z, silu_f32(g3) * v.w)};
         } else {

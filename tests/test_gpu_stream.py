@@ -232,3 +232,38 @@ def test_gate_up_paired_kgroup_tiles(gpu, ff, r, T):
     if T % 8 == 0:
         assert torch.equal(ops.fused_gate_up(xt, *ft[:4], out_transposed=True).t(), h)
     assert _rel(_np(ops.svd_mlp(xt, *ft)), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+
+
+# The gate values stay in 32 bits up to SiLU for ranks off the stages and for
+# transposed results at token counts off 8.  U holds one-hot columns, so XU is
+# exact and h is one rounding to bf16 from 64 bits: its error over the one of a
+# correctly rounded h is the fp32 sums' (1e-5 of it), where a gate value
+# rounded to bf16 on the way would bring sqrt(2) times the error.  fn 4, 7 and
+# 8 tiles (ff = 2048 / 1792), split and unsplit, natural, Linear and fp8.
+@pytest.mark.parametrize("T", [65, 131, 300, 500, 515, 1030])
+@pytest.mark.parametrize("kind,ff,r", [(k, ff, r) for k in ("natural", "linear", "fp8")
+                                       for ff, r in ((2048, 336), (1792, 528), (1800, 80), (2048, 256))
+                                       if k != "fp8" or r % 32])  # fp8: no transposed result at such counts
+def test_gate_values_keep_32_bits(gpu, kind, ff, r, T):
+    out_t = r % 32 == 0
+    d, rng = 640, np.random.default_rng(T + r)
+    u = [np.eye(d, dtype=np.float32)[:, rng.permutation(d)[:r]] for _ in range(2)]
+    v = [inputs.random_matrix(rng, r, ff) for _ in range(2)]
+    xt = torch.from_numpy(rng.normal(size=(T, d)).astype(np.float32)).to(gpu, torch.bfloat16)
+    mats = [torch.from_numpy(np.ascontiguousarray(a)) for a in (u[0], v[0], u[1], v[1])]
+    if kind == "fp8":
+        q = [fp8.quantize_per_channel(a) for a in mats]
+        wide = [torch.from_numpy(O.e4m3_decode(a.data.view(torch.uint8).numpy()) * a.scale.numpy()) for a in q]
+        ft = [ops.QuantizedFactor(a.data.to(gpu), a.scale.to(gpu)) for a in q]
+        wide[0], wide[2] = mats[0], mats[2]
+    else:
+        ft = [a.to(gpu, torch.bfloat16) for a in mats]
+        wide = [a.float().cpu() for a in ft]
+        if kind == "linear":
+            ft = [a.t().contiguous().t() for a in ft]
+    x64, (ug, vg, uu, vu) = xt.double().cpu(), (a.double() for a in wide)
+    g = (x64 @ ug) @ vg
+    want = g * torch.sigmoid(g) * ((x64 @ uu) @ vu)
+    h = ops.fused_gate_up(xt, *ft, out_transposed=True).t() if out_t else ops.fused_gate_up(xt, *ft)
+    err = float((h.cpu().double() - want).norm())
+    assert err < 1.05 * float((want.bfloat16().double() - want).norm())
