@@ -17,8 +17,8 @@ hipError_t go(const BigParams& p, int splits, int batch, hipStream_t st) {
     }
     return hipErrorInvalidValue;
   }
-  if (!C::RM && (p.nmap[0].shift || p.kmap[0].shift)) {  // fp8 B: instances of their own, 8 waves
-    if constexpr (F8 && NW == 8) {
+  if (p.nmap[0].shift || p.kmap[0].shift) {  // instances of their own, 8 waves
+    if constexpr (NW == 8 && !TR && (EPI == BEPI_STORE || EPI == BEPI_DUAL_F32)) {
       hipLaunchKernelGGL(big_gemm_kernel<BigCfgRM<C>>, grid, dim3(C::THREADS), 0, st, p);
       return hipGetLastError();
     }

@@ -238,8 +238,9 @@ struct BigParams {
   // multiple of 64) on moved up by `shift`, zeros in between.  nmap: the X.U
   // product writes it so (output column n >= cut takes B column n - shift,
   // the gap none); kmap: the product that reads it (B rows of stages from cut
-  // on lie `shift` rows earlier: the last 64 rows of V, of which the first
-  // `shift` meet the zeros).  No B row or column outside the matrix is read.
+  // on lie `shift` rows earlier: the last 64 rows of V, the first `shift` of
+  // which were taken before and are fetched as zeros, so that an infinity in
+  // them counts once).  No B row or column outside the matrix is read.
   RankMap nmap[2], kmap[2];
   // Gate values in 32 bits (G32 instances; null: bf16): gmem then holds their
   // upper halves and glo, the h buffer itself, their lower ones, each lane's
@@ -266,10 +267,13 @@ struct BigCfg {
   // instance: its block-to-tile arithmetic, compiled into every instance,
   // cost the fp8-B ones ~20 VGPRs and the 256 x 256 fp8-B ones a spill.
   static constexpr bool TR = TR_;
-  // RM: the launch may carry rank maps (BigParams::nmap, kmap).  The fp8
-  // instances have it apart (BigCfgRM): in their loop it cost the 70B layer
-  // 0.5% (the bf16 ones measure the same with and without).
-  static constexpr bool RM = !FP8_B_;
+  // RM: the launch may carry rank maps (BigParams::nmap, kmap), on instances
+  // of their own (BigCfgRM): in the loop of the fp8 ones they cost the 70B
+  // layer 0.5%.  Leaving out the repeated rows by the uniform descriptor costs
+  // no register (8B layer at rank 2744, T=512 / 1024: 214.8 / 329.8 us, 214.7 /
+  // 330.4 with the rows multiplied by zero); by a per-lane offset the 256 x
+  // 256 dual instances spill.
+  static constexpr bool RM = false;
   static constexpr bool G32 = false;  // gate values in 32 bits between the passes (BigCfgG32)
   static constexpr int WT = NW / KG;                 // wave tiles per block
   static constexpr int THREADS = 64 * NW;
@@ -473,7 +477,19 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         const int i = d - C::A_UNITS;
         const uint32_t kr = (uint32_t)(C::RM && k0 >= km.cut ? k0 - km.shift : k0);
         const uint32_t soff = C::B_KC ? kr * 2u : (C::FP8_B ? kr * (uint32_t)ldb : kr * ldb2);
-        dma16(live ? rb : r_none, b_voff[i], soff, lbase + B_REGION + s * C::B_BYTES + (wave + NW * i) * 1024);
+        // the stage's first `gone` k were taken before (RankMap): a multiple of
+        // 8, so that whole instructions (2 or 4 natural-layout rows) or whole
+        // pieces (8 k of a Linear row, part of a 384-byte one) are left out
+        const int gone = C::RM && k0 >= km.cut ? km.cut + km.shift - k0 : 0;
+        i32x4 rs = live ? rb : r_none;
+        uint32_t voff = b_voff[i];
+        if constexpr (C::RM && C::B_KC)
+          voff = 8 * ((lane & 3) ^ a_swz(16 * wave + (lane >> 2))) < gone ? kOOB : voff;
+        else if constexpr (C::RM && C::B_PITCH == 384)
+          voff = (wave + NW * i) * 1024 + 16 * lane < gone * 384 ? kOOB : voff;
+        else if constexpr (C::RM)
+          rs[2] = 1024 / C::B_PITCH * (wave + NW * i) >= gone ? rs[2] : 0;  // no records
+        dma16(rs, voff, soff, lbase + B_REGION + s * C::B_BYTES + (wave + NW * i) * 1024);
       }
     };
     constexpr int NDMA = C::A_UNITS + C::B_UNITS;

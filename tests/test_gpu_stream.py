@@ -218,6 +218,27 @@ def test_ranks_off_the_stages(gpu, shape, kind, T):
         assert _rel(_np(blk), _np((xt.float() + ops.svd_mlp(xn, *ft).float()).bfloat16())) < TOL
 
 
+# An infinite weight among the rows that the last 64-rank block repeats gives
+# infinities by the sign of its rank value, not NaN (infinity times zero).
+@pytest.mark.parametrize("T", [65, 300, 1030])
+@pytest.mark.parametrize("kind", ["natural", "linear"])
+@pytest.mark.parametrize("r", [72, 336, 504])
+def test_ranks_off_the_stages_infinite_weight(gpu, r, kind, T):
+    d, ff = 512, 1024
+    rng = np.random.default_rng(T + r)
+    u = torch.from_numpy(np.eye(d, dtype=np.float32)[:, :r].copy()).to(gpu, torch.bfloat16)
+    v = torch.from_numpy(inputs.random_matrix(rng, r, ff)).to(gpu, torch.bfloat16)
+    v[r - 64, 5] = float("inf")
+    v[(r - 1) // 64 * 64 - 1, 700] = float("-inf")
+    x = torch.from_numpy(rng.choice([-1.5, 0.75, 2.0], size=(T, d)).astype(np.float32)).to(gpu, torch.bfloat16)
+    want = x.float().cpu()[:, :r] @ v.float().cpu()
+    if kind == "linear":
+        u, v = u.t().contiguous().t(), v.t().contiguous().t()
+    got = ops.fused_xuv(x, u, v).float().cpu()
+    assert torch.equal(torch.isposinf(got), torch.isposinf(want)) and torch.equal(torch.isneginf(got), torch.isneginf(want))
+    assert torch.isfinite(got).sum() == T * (ff - 2)
+
+
 # 129-256 tokens where the 128 x 128 K-group tiles fill at most half the CUs:
 # the branches as batch entries in 1, 2 and 4 K splits (the last one ragged at
 # rank 1088 and 2112), ragged last row tiles, the transposed result, a rank at
