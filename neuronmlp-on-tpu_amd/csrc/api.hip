@@ -19,7 +19,8 @@
 //                                    with too few output tiles split K into
 //                                    fp32 slices summed in split order
 //   1-64 tokens, Linear-layout or fp8 factors, dimensions off the decode
-//   layer's tiles (multiples of 8), and the gate/up and x.u.v entry points:
+//   layer's tiles (multiples of 8), and the gate/up and x.u.v entry points;
+//   65-128 where the factors are small or off the large tiles (decode_ok):
 //                                    one streaming launch per stage (stream.hpp)
 //   fp32, aligned:                   one fp32 streaming launch per stage
 //                                    (stream_f32.hpp)
@@ -481,6 +482,7 @@ struct Tune {
   // decode layer: most K splits of phases 1, 3, 4 (0: grid / tiles; -1: the
   // defaults, dls3 8 at two token tiles, dls4 4 at four, else grid / tiles)
   int dls1 = 0, dls3 = -1, dls4 = -1;
+  int strfp8 = 64, strlin = 48;  // streaming stages at 65-128 tokens: largest factor pair (MB)
   int p2k = -1;        // decode layer: smallest K of a phase-2 split (0: no splits, -1: p2_splits' own)
   bool dlpff = true;   // decode layer: the weight prefetch at a grid barrier fills the whole ring
   bool dlready = true;  // decode layer: phase 4 waits for its XU_d tiles' ready flags, not a grid barrier
@@ -570,6 +572,8 @@ const Tune& tune() {
         if (k == "kgw") r.kgw = v;
         if (k == "kgs") r.kgs = v;
         if (k == "p2k") r.p2k = v;
+        if (k == "strfp8") r.strfp8 = v;
+        if (k == "strlin") r.strlin = v;
         if (k == "dls1") r.dls1 = v;
         if (k == "dls3") r.dls3 = v;
         if (k == "dls4") r.dls4 = v;
@@ -1454,11 +1458,12 @@ int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, boo
   int ks = 0;
   p.T = (int)T;
   for (int i = 0; i < nseg; ++i) p.tiles += !dual || i == 0 ? (int)((N[i] + bn - 1) / bn) : 0;
+  p.groups = (int)((T + kStRows - 1) / kStRows);
   size_t off = 0;
   const int64_t area = stream_area(L, ws_bytes, &off);
   p.slices = reinterpret_cast<float*>(ws + off);
   p.slice_bytes = (uint32_t)area;
-  p.splits = stream_splits(K, p.tiles, (dual ? 2 : 1) * T * bn * 4, area, &ks);
+  p.splits = stream_splits(K, p.groups * p.tiles, (dual ? 2 : 1) * std::min<int64_t>(T, kStRows) * bn * 4, area, &ks);
   p.exchange = p.splits > 1 || out[0].t;
   p.out_t = out[0].t;
   p.sync = reinterpret_cast<uint64_t*>(ws + L.sync);
@@ -1474,16 +1479,31 @@ int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, boo
 // A streaming stage can write its tiles transposed: each then goes through
 // the slice area whole.
 bool stream_out_t_ok(int64_t T, int64_t N, const Ws& L, size_t ws_bytes) {
-  const int64_t tiles = (N + 2 * kStTileN - 1) / (2 * kStTileN) * 2;
+  const int64_t tiles = (N + 2 * kStTileN - 1) / (2 * kStTileN) * 2 * ((T + kStRows - 1) / kStRows);
   size_t off = 0;
-  return tiles <= kDlMaxTiles && tiles * 2 * T * kStTileN * 4 <= stream_area(L, ws_bytes, &off);
+  return tiles <= kDlMaxTiles && tiles * 2 * std::min<int64_t>(T, kStRows) * kStTileN * 4 <= stream_area(L, ws_bytes, &off);
 }
 
 // Streaming stages take bf16 activations and any bf16 or fp8 factors in rows
 // of whole 16-byte pieces (fp8: 8), with the 32-bit offsets of one step and of
 // the activations in range.
-bool decode_ok(const Common& c, int64_t T, std::initializer_list<int64_t> dims, bool vec) {
-  if (c.f32 || T > kDecodeMaxT || !vec) return false;
+//
+// At 65-128 tokens, in two row groups that each stream the factors, they beat
+// the large tiles (10 us of pipeline fill and epilogue a launch, slices and
+// their reductions) while a pair U, V (r (d + ff) values) is small, and take
+// what the large tiles do not (`big` false: 8B fp8 layer at rank 2744, T=128,
+// 840 -> 134 us).  us per layer at T=65 / 128, large tiles -> streamed: fp8
+// (4096, 14336, 2816), 52 MB a pair, 154 / 154 -> 110 / 127; (3072, 8192, 1792)
+// 121 / 123 -> 73 / 78, (1024, 3584, 256) 91 / 91 -> 48 / 48; at 207 MB (70B)
+// 315 / 333 -> 341 / 406.  Linear: (3072, 8192, 1792), 40 MB, 108 / 105 -> 92 /
+// 97, (2048, 5632, 1152) 95 / 91 -> 70 / 73; at 104 MB (8B) 153 / 158 -> 172 /
+// 183.  Natural bf16 stays on the K-group tiles: (3072, 8192, 1736) 81 / 82 us
+// there, 80 / 89 streamed (smaller layers gain a little, 17 MB 68 / 66 -> 62 / 64).
+bool decode_ok(const Common& c, int64_t T, std::initializer_list<int64_t> dims, bool vec, bool lin, int64_t pair, bool big) {
+  if (c.f32 || !vec || T > kStMaxT) return false;
+  const bool f8 = c.wt == SVDMLP_FP8_E4M3;
+  if (T > kDecodeMaxT && big && pair * wbytes(c) > (int64_t)(f8 ? tune().strfp8 : lin ? tune().strlin : 0) * 1000000)
+    return false;
   for (int64_t v : dims)
     if (v % 8 || v >= (int64_t)1 << 22 || T * v * 2 >= ((int64_t)1 << 31)) return false;
   return true;
@@ -2075,7 +2095,8 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
   if (fp8 && (!vec || (out_t && T % 8))) return fail("fp8 weights need d, ff and r to be multiples of 8 and 16-byte aligned buffers");
   char* ws = static_cast<char*>(workspace);
 
-  if (decode_ok(c, T, {d, ff, r}, vec)) {
+  const bool big = big_ok(c, vec, {T * d * 2, d * r * 2, r * ff * 2, T * ff * 2}, {d}) && big_rank_ok(c, r);
+  if (decode_ok(c, T, {d, ff, r}, vec, u_lin && v_lin, r * (d + ff), big)) {
     uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
     const uint16_t* x16 = static_cast<const uint16_t*>(x);
     {
@@ -2101,7 +2122,7 @@ int svdmlp_gate_up(const void* x, const void* ug, const void* vg, const void* uu
     return check(launch_transpose_bf16(hn, ff, static_cast<uint16_t*>(h), T, (int)T, (int)ff, c.st), "h transpose");
   }
 
-  if (big_ok(c, vec, {T * d * 2, d * r * 2, r * ff * 2, T * ff * 2}, {d}) && big_rank_ok(c, r)) {
+  if (big) {
     const void* us[2] = {ug, uu};
     const float* sus[2] = {s_ug, s_uu};
     if ((rc = big_xu(c, ST_GU_XU, x, d, T * d * 2, us, u_lin, T, d, r, 2, ws, L, fp8 ? sus : nullptr))) return rc;
@@ -2174,7 +2195,8 @@ int svdmlp_xuv(const void* x, const void* u, const void* v, const float* s_u, co
     x_t = false;
   }
 
-  if (!x_t && decode_ok(c, T, {din, dout, r}, vec)) {
+  const bool big = !x_t && big_ok(c, vec, {T * din * 2, din * r * 2, r * dout * 2, T * dout * 2}, {din}) && big_rank_ok(c, r);
+  if (!x_t && decode_ok(c, T, {din, dout, r}, vec, u_lin && v_lin, r * (din + dout), big)) {
     uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
     const uint16_t* a1 = static_cast<const uint16_t*>(x);
     const StreamOut o1{xu, r}, o2{static_cast<uint16_t*>(y), dout};
@@ -2186,7 +2208,7 @@ int svdmlp_xuv(const void* x, const void* u, const void* v, const float* s_u, co
                         "decode XU.V");
   }
 
-  if (!x_t && big_ok(c, vec, {T * din * 2, din * r * 2, r * dout * 2, T * dout * 2}, {din}) && big_rank_ok(c, r)) {
+  if (big) {
     const void* us[1] = {u};
     const float* sus[1] = {s_u};
     if ((rc = big_xu(c, ST_D_XU, x, din, T * din * 2, us, u_lin, T, din, r, 1, ws, L, fp8 ? sus : nullptr)))
@@ -2383,7 +2405,8 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
                 "multiples of 128, 128 and 64, the large-tile path more than %lld tokens)", (long long)kDecodeMaxT);
   if ((rc = normed())) return rc;
 
-  if (decode_ok(c, T, {d, ff, r_gu, r_d}, vec)) {
+  // (padded factors and e4m3 h above the decode token counts are the large tiles')
+  if (ld.dense && !(fp8_act && T > kDecodeMaxT) && decode_ok(c, T, {d, ff, r_gu, r_d}, vec, u_lin && v_lin, std::max(r_gu, r_d) * (d + ff), big)) {
     uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
     uint16_t* hb = reinterpret_cast<uint16_t*>(ws + L.h);
     const uint16_t* x16 = static_cast<const uint16_t*>(x);

@@ -1,6 +1,8 @@
 // Instances and launcher of the decode-shape streaming stages (stream.hpp).
 #include "stream.hpp"
 
+#include <algorithm>
+
 #include "dispatch.hpp"
 
 namespace svdmlp {
@@ -9,7 +11,7 @@ namespace {
 
 template <int MT, int WK, int CG = 1>
 hipError_t go(const StreamParams& p, bool dual, hipStream_t st) {
-  const dim3 grid(p.tiles * p.splits);
+  const dim3 grid(p.tiles * p.splits, p.groups);
   if (dual)
     hipLaunchKernelGGL((stream_kernel<MT, WK, CG, true>), grid, dim3(kStThreads), 0, st, p);
   else
@@ -30,11 +32,11 @@ hipError_t go_w(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st
 
 hipError_t launch_stream(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st, const char** why) {
   if (p.T < 1 || p.T > kStMaxT || p.tiles < 1 || p.splits < 1 || (p.splits > 1 && !p.exchange) ||
-      (p.splits > 1 && p.tiles > kDlMaxTiles) || (cg != 1 && (wk != SW_FP8 || cg != 2 || p.T > 32))) {
+      (p.splits > 1 && p.groups * p.tiles > kDlMaxTiles) || p.groups != (p.T + kStRows - 1) / kStRows || (cg != 1 && (wk != SW_FP8 || cg != 2 || p.T > 32))) {
     *why = "streaming stage: token count, tiles, splits or column groups outside the kernel's range";
     return hipErrorInvalidValue;
   }
-  if (p.exchange && (int64_t)p.tiles * p.splits * (dual ? 2 : 1) * cg * p.T * kStTileN * 4 > (int64_t)p.slice_bytes) {
+  if (p.exchange && (int64_t)p.groups * p.tiles * p.splits * (dual ? 2 : 1) * cg * std::min(p.T, kStRows) * kStTileN * 4 > (int64_t)p.slice_bytes) {
     *why = "streaming stage: the K splits' slices exceed the workspace's area";
     return hipErrorInvalidValue;
   }

@@ -1,4 +1,4 @@
-// Decode-shape (T <= 64 tokens) projections as one launch per stage: weight
+// Decode-shape (T <= 128 tokens) projections as one launch per stage: weight
 // streaming at HBM rate for the operands the persistent decode layer does not
 // take (Linear-layout and fp8 factors, dimensions off its tiles) and for the
 // gate/up and x.u.v entry points, which run only half of the layer.
@@ -38,8 +38,10 @@
 // TB/s), 8B Linear-layout layer at 16 tokens 170 -> 82 us, 8B x.u.v at 32
 // tokens 114 -> 33 us.  What is left per launch is ~3.5-4.5 us of launch,
 // ramp and in-block sums and 1.5 us (16 tokens) to 4 us (64) of slices.
-// Above 64 tokens the large-tile path is faster (8B gate/up at 65 / 128
-// tokens 71 / 77 us against 79 / 98 with two row groups of waves here).
+// At 65-128 tokens two groups of 64 rows run side by side as blocks of their
+// own, each streaming the weights (they meet in L2), so the time grows with
+// the factors where the large tiles' is mostly fixed: decode_ok (api.hip) has
+// the line between them.
 #pragma once
 
 #include "gemm_big.hpp"
@@ -64,6 +66,7 @@ struct StreamSeg {
 struct StreamParams {
   StreamSeg seg[2];       // DUAL: gate and up branch of one output (seg[0].out)
   int T, splits, tiles;   // tiles: column tiles over the segments (DUAL: of one)
+  int groups;             // ceil(T / 64) groups of 64 token rows, each with units of its own
   int exchange;           // units meet through slices (more than one split, or out_t)
   int out_t;              // out is (N, T): T a multiple of 8
   float* slices;          // fp32, (tile, split, branch) slices of T x 128
@@ -72,7 +75,8 @@ struct StreamParams {
   const uint16_t* resid;  // (T, N) added to bf16(out), row pitch ldo, or null
 };
 
-constexpr int kStMaxT = 64;
+constexpr int kStRows = 64;  // token rows of a group
+constexpr int kStMaxT = 2 * kStRows;
 constexpr int kStThreads = 512;
 constexpr int kStTileN = 128;
 constexpr uint32_t kStNone = 0xfffffff0u;  // past the slice area: reads zeros
@@ -107,11 +111,11 @@ __device__ __forceinline__ uint32_t st_fp8_pair(uint32_t d, bool high) {
 // outside as a whole): kOOB reads zeros whichever way the scalar offset
 // enters the range check.
 template <int MT, int WK, int CG>
-__device__ __forceinline__ void st_load(const StreamSeg& s, int T, int n0, int k0, bool live, int lr, int lg,
-                                        StStep<MT, WK, CG>& r) {
+__device__ __forceinline__ void st_load(const StreamSeg& s, const uint16_t* a, int T, int n0, int k0, bool live, int lr,
+                                        int lg, StStep<MT, WK, CG>& r) {
   const int records = live ? 0x7ffffff0 : 0;
   const __amdgpu_buffer_rsrc_t ra =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(s.a) + k0, 0, records, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a) + k0, 0, records, 0x00020000);
   constexpr int esz = WK == SW_FP8 ? 1 : 2;
   const char* wb = static_cast<const char*>(s.w) +
                    (WK == SW_LINEAR ? (int64_t)n0 * s.ldw + k0 : (int64_t)k0 * s.ldw + n0) * esz;
@@ -188,7 +192,9 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   __shared__ int last;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane & 15, lg = lane >> 4;
-  const int T = p.T;
+  const int m00 = blockIdx.y * kStRows;     // the group's first token row
+  const int T = min(p.T - m00, kStRows);    // and its rows
+  const uint32_t srows = min(p.T, kStRows);  // rows of a slice
   // A workspace whose persistent decode call timed out has counters in an
   // unknown state: NaN until it is reset, as the decode layers write.
   const bool poison = __hip_atomic_load(&p.sync[kDlFlag], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
@@ -201,6 +207,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const int n0 = (second ? tile - p.seg[0].ntiles : tile) * kStTileN * CG;
   const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
+  const uint16_t* const a = s.a + (int64_t)m00 * s.K;
 
   f32x4 acc[CG][MT][8];
 #pragma unroll
@@ -217,7 +224,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   StStep<MT, WK, CG> r0, r1;
   auto load = [&](int i, StStep<MT, WK, CG>& r) {
     const int k = kb + 64 * (i / S * NWB + wb) + 32 * (i % S);
-    st_load<MT, WK, CG>(s, T, n0, k, i < steps && k < ke, lr, lg, r);
+    st_load<MT, WK, CG>(s, a, T, n0, k, i < steps && k < ke, lr, lg, r);
   };
   load(0, r0);
   for (int i = 0; i < steps; i += 2) {
@@ -243,14 +250,14 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
     }
     u32x2 o = u32x2{pack_bf16x2(v0.x, v0.y), pack_bf16x2(v0.z, v0.w)};
     if (p.resid) {
-      const u32x2 x = *reinterpret_cast<const u32x2*>(p.resid + (int64_t)m * so.ldo + col);
+      const u32x2 x = *reinterpret_cast<const u32x2*>(p.resid + (int64_t)(m00 + m) * so.ldo + col);
       o = u32x2{add_bf16x2(x.x, o.x), add_bf16x2(x.y, o.y)};
     }
     constexpr uint32_t kNaN2 = 0x7fc07fc0u;
     return poison ? u32x2{kNaN2, kNaN2} : o;
   };
   auto store = [&](int m, int n, u32x2 v) {
-    *reinterpret_cast<u32x2*>(so.out + (int64_t)m * so.ldo + n0 + n) = v;
+    *reinterpret_cast<u32x2*>(so.out + (int64_t)(m00 + m) * so.ldo + n0 + n) = v;
   };
 
   // ---- the 8 waves' sums, 16 token rows at a time: thread (row tid / 32,
@@ -259,7 +266,8 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   // that the lanes of a pass cover all 64 banks. ----
   const int qm = tid >> 5, qn = 4 * (tid & 31);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(p.slices, 0, (int)p.slice_bytes, 0x00020000);
-  const uint32_t unit = (uint32_t)(tile * p.splits + split) * BR;
+  const int gtile = blockIdx.y * p.tiles + tile;  // the tile's counter
+  const uint32_t unit = (uint32_t)(gtile * p.splits + split) * BR;
 #pragma unroll
   for (int g = 0; g < CG; ++g) {
     const int n = column(g, qn);
@@ -289,7 +297,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
             for (int b = 0; b < BR; ++b)
               __builtin_amdgcn_raw_buffer_store_b128(
                   u32x4{__float_as_uint(v[b].x), __float_as_uint(v[b].y), __float_as_uint(v[b].z), __float_as_uint(v[b].w)},
-                  rs, ((((unit + b) * CG + g) * (uint32_t)T + (uint32_t)m) * kStTileN + (uint32_t)qn) * 4u, 0, kDlSc1);
+                  rs, ((unit + b) * CG * srows + (uint32_t)(g * T + m)) * (kStTileN * 4u) + 4u * (uint32_t)qn, 0, kDlSc1);
           }
         }
       }
@@ -303,13 +311,13 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   __syncthreads();
   if (tid == 0)
     last = poison || p.splits == 1 ||
-           __builtin_amdgcn_atomic_inc32(dl_tile_counter(p.sync, tile), (uint32_t)p.splits - 1u, __ATOMIC_RELAXED, "agent") ==
+           __builtin_amdgcn_atomic_inc32(dl_tile_counter(p.sync, gtile), (uint32_t)p.splits - 1u, __ATOMIC_RELAXED, "agent") ==
                (uint32_t)p.splits - 1u;
   __syncthreads();
   if (!last) return;
   uint16_t* const tl = reinterpret_cast<uint16_t*>(&red[0][0]);  // out_t: the tile as [column][token]
   const int tp = T + 8;
-  const uint32_t unit0 = (uint32_t)(tile * p.splits) * BR;
+  const uint32_t unit0 = (uint32_t)(gtile * p.splits) * BR;
   constexpr int SB = DUAL ? 4 : 8;  // splits in flight
   for (int q = tid; q < T * 32 * CG; q += kStThreads) {  // (group, token, column quad), in slice order
     const int g = CG == 1 ? 0 : q / (T * 32), m = (q >> 5) - g * T, n = column(g, 4 * (q & 31));
@@ -322,7 +330,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
 #pragma unroll
         for (int b = 0; b < BR; ++b)
           x[k][b] = __builtin_amdgcn_raw_buffer_load_b128(
-              rs, s0 + k < p.splits ? (unit0 + (uint32_t)((s0 + k) * BR + b)) * (uint32_t)(T * CG * kStTileN * 4) + 16u * (uint32_t)q
+              rs, s0 + k < p.splits ? (unit0 + (uint32_t)((s0 + k) * BR + b)) * (srows * (uint32_t)(CG * kStTileN * 4)) + 16u * (uint32_t)q
                                     : kStNone,
               0, kDlSc1);
 #pragma unroll
@@ -348,7 +356,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   for (int q = tid; q < kStTileN * CG * per; q += kStThreads) {
     const int n = q / per, i = q % per;
     if (n0 + n < so.N)
-      *reinterpret_cast<u32x4*>(so.out + (int64_t)(n0 + n) * so.ldo + 8 * i) = *reinterpret_cast<const u32x4*>(tl + n * tp + 8 * i);
+      *reinterpret_cast<u32x4*>(so.out + (int64_t)(n0 + n) * so.ldo + m00 + 8 * i) = *reinterpret_cast<const u32x4*>(tl + n * tp + 8 * i);
   }
 }
 

@@ -71,6 +71,46 @@ def test_stream_entry_points(gpu, shape, kind, T):
         assert torch.equal(yT.view(torch.int16), y.view(torch.int16))
 
 
+# 65-128 tokens: a second group of token rows with units, slices and tile
+# counters of its own, from one row to full; K splits (d = 4160) and none,
+# dimensions that the large tiles take (512, 1024) and not, the transposed
+# result, the block's residual.
+@pytest.mark.parametrize("T", [65, 72, 113, 128])
+@pytest.mark.parametrize("kind", ["natural", "linear", "fp8"])
+@pytest.mark.parametrize("shape", [inputs.LayerShape(136, 200, 72, 40), inputs.LayerShape(4160, 528, 136, 264),
+                                   inputs.LayerShape(264, 2064, 400, 272), inputs.LayerShape(512, 1024, 160)])
+def test_stream_two_row_groups(gpu, shape, kind, T):
+    xb, wide, xt, ft = _layer(shape, T, 900 + T, kind, gpu)
+    h = ops.fused_gate_up(xt, *ft[:4])
+    assert _rel(_np(h), O.fused_gate_up_ref(xb, *wide[:4], dtype="bfloat16")) < TOL
+    y = ops.fused_xuv(h, *ft[4:])
+    assert _rel(_np(y), O.fused_xuv_ref(_np(h), *wide[4:], dtype="bfloat16")) < TOL
+    ops.clear_workspace_cache()
+    out = ops.svd_mlp(xt, *ft)
+    assert _rel(_np(out), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+    for _ in range(3):
+        assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
+    (ws,) = ops._WS_CACHE.values()
+    assert not any(ws[2560:4096].view(torch.int32).cpu().tolist())
+    if T % 8 == 0 or kind != "fp8":
+        hT = ops.fused_gate_up(xt, *ft[:4], out_transposed=True)
+        assert torch.equal(hT.view(torch.int16), h.t().contiguous().view(torch.int16))
+        yT = ops.fused_xuv(h.t().contiguous(), *ft[4:], x_transposed=True)
+        assert torch.equal(yT.view(torch.int16), y.view(torch.int16))
+    gain = torch.rand(shape.d, device=gpu) + 0.5
+    xn = (xt.float() * torch.rsqrt(xt.float().pow(2).mean(1, keepdim=True) + 1e-5) * gain).bfloat16()
+    want = (xt.float() + ops.svd_mlp(xn, *ft).float()).bfloat16()
+    assert _rel(_np(ops.svd_mlp_block(xt, gain, *ft)), _np(want)) < TOL
+
+
+def test_stream_two_row_groups_leave_padded_factors(gpu):
+    """Factors with padded rows stay on the large tiles, which know the pitch."""
+    xb, wide, xt, ft = _layer(inputs.LayerShape(512, 1024, 160), 100, 15, "natural", gpu)
+    padded = [ops.pad_rows(a) if i % 2 else a for i, a in enumerate(ft)]
+    assert padded[1].stride(0) > padded[1].shape[1]
+    assert _rel(_np(ops.svd_mlp(xt, *padded)), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+
+
 @pytest.mark.parametrize("kind", ["linear", "fp8"])
 def test_stream_block(gpu, kind):
     """The MLP block: RMSNorm ahead, the residual added by the last stage."""
