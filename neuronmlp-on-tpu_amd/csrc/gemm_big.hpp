@@ -717,6 +717,9 @@ __global__ __launch_bounds__(C::THREADS, 1) void big_gemm_kernel(BigParams p) {
         if constexpr (C::FP8_B)
           // per-column dequant (fp8 ranks keep the map's bounds at multiples of 16: the column's is a scalar)
           if (n < N) v *= *reinterpret_cast<const f32x4*>(p.scale[zb] + (C::RM ? b_col(n0 + wn0 + 16 * j) + 4 * lg : n));
+        // columns in the rank map's gap are zeros whatever A holds (its zero B
+        // columns times an infinite A are NaN, which zero B rows would keep)
+        if constexpr (C::RM && C::EPI == BEPI_STORE) v = b_has(n) ? v : f32x4{0.f, 0.f, 0.f, 0.f};
         const int64_t fo = frag0 + (int64_t)(i * FN + j) * 256;
         if constexpr (FRAG) {
           // (a dual block's gate values go to gmem, its own buffer)

@@ -279,6 +279,34 @@ def test_ranks_off_the_stages_infinite_weight(gpu, r, kind, T):
     assert torch.isfinite(got).sum() == T * (ff - 2)
 
 
+# An infinite activation: the rank columns that the last 64-rank block repeats
+# hold zeros for XU's gap, not the NaN of infinity times a zero weight.  U and
+# V of one sign keep the results infinite.  Split and unsplit X.U products of
+# every tile width, natural and Linear factors.
+@pytest.mark.parametrize("T", [65, 130, 300, 1030])
+@pytest.mark.parametrize("kind", ["natural", "linear", "fp8"])
+@pytest.mark.parametrize("r", [80, 336, 504, 1104])
+def test_ranks_off_the_stages_infinite_activation(gpu, r, kind, T):
+    d, ff = 512, 1024
+    rng = np.random.default_rng(T + r)
+    f = [torch.from_numpy(np.abs(inputs.random_matrix(rng, *s)) + 0.01) for s in ((d, r), (r, ff), (d, r), (r, ff), (ff, r), (r, d))]
+    x = torch.from_numpy(np.abs(rng.normal(size=(T, d))).astype(np.float32))
+    rows = [3, T // 2, T - 1]
+    for i, m in enumerate(rows):
+        x[m, 7 * i] = float("inf")
+    x = x.to(gpu, torch.bfloat16)
+    if kind == "fp8":
+        f = [fp8.quantize_per_channel(a.to(gpu)) for a in f]
+    else:
+        f = [a.to(gpu, torch.bfloat16) for a in f]
+        if kind == "linear":
+            f = [a.t().contiguous().t() for a in f]
+    for got in (ops.fused_xuv(x, f[0], f[1]), ops.fused_gate_up(x, *f[:4]), ops.svd_mlp(x, *f)):
+        got = got.float().cpu()
+        inf = torch.isposinf(got)
+        assert inf[rows].all() and torch.isfinite(got).sum() == got.numel() - inf[rows].numel()
+
+
 # 129-256 tokens where the 128 x 128 K-group tiles fill at most half the CUs:
 # the branches as batch entries in 1, 2 and 4 K splits (the last one ragged at
 # rank 1088 and 2112), ragged last row tiles, the transposed result, a rank at
