@@ -323,6 +323,7 @@ struct Common {
   bool f32;
   hipStream_t st;
   Block* blk = nullptr;
+  bool layer = false;  // a call of the whole layer (or block), not of one half
 };
 
 int check_types(int32_t act, int32_t wt) {
@@ -1464,10 +1465,10 @@ int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, boo
   p.slices = reinterpret_cast<float*>(ws + off);
   p.slice_bytes = (uint32_t)area;
   p.splits = stream_splits(K, p.groups * p.tiles, (dual ? 2 : 1) * std::min<int64_t>(T, kStRows) * bn * 4, area, &ks);
-  p.exchange = p.splits > 1 || out[0].t;
   p.out_t = out[0].t;
   p.sync = reinterpret_cast<uint64_t*>(ws + L.sync);
   p.resid = out[0].resid;
+  p.layer = c.layer;
   for (int i = 0; i < nseg; ++i)
     p.seg[i] = StreamSeg{a[i], w[i], sw ? sw[i] : nullptr, out[dual ? 0 : i].p, w_lin ? K : N[i], out[dual ? 0 : i].ld,
                          (int)K, (int)N[i], (int)((N[i] + bn - 1) / bn), ks};
@@ -2284,7 +2285,7 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
   const int64_t r = std::max(std::max(r_g, r_u), r_d);
   const Ws L = ws_layout(T, d, ff, r);
   if (ws_bytes < L.need) return fail("workspace too small: need %zu bytes, got %zu", L.need, ws_bytes);
-  const Common c{act_dtype, w_dtype, act_dtype == SVDMLP_F32, (hipStream_t)stream, blk};
+  const Common c{act_dtype, w_dtype, act_dtype == SVDMLP_F32, (hipStream_t)stream, blk, true};
   const bool u_lin = flags & SVDMLP_U_LINEAR, v_lin = flags & SVDMLP_V_LINEAR;
   bool vec = d % 8 == 0 && ff % 8 == 0 && r_g % 8 == 0 && r_u % 8 == 0 && r_d % 8 == 0;
   for (const void* q : {x, ug, vg, uu, vu, ud, vd, (const void*)y, (const void*)workspace}) vec = vec && aligned16(q);

@@ -31,12 +31,12 @@ hipError_t go_w(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st
 }  // namespace
 
 hipError_t launch_stream(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st, const char** why) {
-  if (p.T < 1 || p.T > kStMaxT || p.tiles < 1 || p.splits < 1 || (p.splits > 1 && !p.exchange) ||
-      (p.splits > 1 && p.groups * p.tiles > kDlMaxTiles) || p.groups != (p.T + kStRows - 1) / kStRows || (cg != 1 && (wk != SW_FP8 || cg != 2 || p.T > 32))) {
+  if (p.T < 1 || p.T > kStMaxT || p.tiles < 1 || p.splits < 1 || p.groups != (p.T + kStRows - 1) / kStRows ||
+      (p.splits > 1 && p.groups * p.tiles > kDlMaxTiles) || (cg != 1 && (wk != SW_FP8 || cg != 2 || p.T > 32))) {
     *why = "streaming stage: token count, tiles, splits or column groups outside the kernel's range";
     return hipErrorInvalidValue;
   }
-  if (p.exchange && (int64_t)p.groups * p.tiles * p.splits * (dual ? 2 : 1) * cg * std::min(p.T, kStRows) * kStTileN * 4 > (int64_t)p.slice_bytes) {
+  if ((p.splits > 1 || p.out_t) && (int64_t)p.groups * p.tiles * p.splits * (dual ? 2 : 1) * cg * std::min(p.T, kStRows) * kStTileN * 4 > (int64_t)p.slice_bytes) {
     *why = "streaming stage: the K splits' slices exceed the workspace's area";
     return hipErrorInvalidValue;
   }

@@ -67,12 +67,12 @@ struct StreamParams {
   StreamSeg seg[2];       // DUAL: gate and up branch of one output (seg[0].out)
   int T, splits, tiles;   // tiles: column tiles over the segments (DUAL: of one)
   int groups;             // ceil(T / 64) groups of 64 token rows, each with units of its own
-  int exchange;           // units meet through slices (more than one split, or out_t)
   int out_t;              // out is (N, T): T a multiple of 8
   float* slices;          // fp32, (tile, split, branch) slices of T x 128
   uint32_t slice_bytes;
   uint64_t* sync;         // tile counters (sync_area.hpp) and the timeout flag
   const uint16_t* resid;  // (T, N) added to bf16(out), row pitch ldo, or null
+  int layer;              // a stage of the layer: NaN while the timeout flag is set
 };
 
 constexpr int kStRows = 64;  // token rows of a group
@@ -195,9 +195,12 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const int m00 = blockIdx.y * kStRows;     // the group's first token row
   const int T = min(p.T - m00, kStRows);    // and its rows
   const uint32_t srows = min(p.T, kStRows);  // rows of a slice
-  // A workspace whose persistent decode call timed out has counters in an
-  // unknown state: NaN until it is reset, as the decode layers write.
-  const bool poison = __hip_atomic_load(&p.sync[kDlFlag], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  // A workspace whose persistent decode call timed out has tile counters in an
+  // unknown state.  The layer then gives NaN until it is reset, as the
+  // persistent layers do; the halves, which no wait precedes, run without the
+  // counters: the first split's unit takes its tile's whole K.  The flag's load
+  // is in flight with the weights' and looked at after them.
+  uint64_t flag = p.sync[kDlFlag];
 
   const int split = blockIdx.x / p.tiles;
   const int tile = blockIdx.x % p.tiles;
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const StreamSeg& so = p.seg[second ? 1 : 0];                        // the output's segment
   const StreamSeg& s = p.seg[DUAL ? wave >> 2 : (second ? 1 : 0)];  // the segment this wave streams
   const int n0 = (second ? tile - p.seg[0].ntiles : tile) * kStTileN * CG;
-  const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
+  int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
   const uint16_t* const a = s.a + (int64_t)m00 * s.K;
 
@@ -219,24 +222,35 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
 
   // step i of this wave: part i % S of its (i / S)-th 64-k block
   constexpr int S = 2 / StStep<MT, WK, CG>::H;
-  const int nblk = (ke - kb + 63) / 64;
-  const int steps = nblk > wb ? (nblk - wb + NWB - 1) / NWB * S : 0;
-  StStep<MT, WK, CG> r0, r1;
-  auto load = [&](int i, StStep<MT, WK, CG>& r) {
-    const int k = kb + 64 * (i / S * NWB + wb) + 32 * (i % S);
-    st_load<MT, WK, CG>(s, a, T, n0, k, i < steps && k < ke, lr, lg, r);
-  };
-  load(0, r0);
-  for (int i = 0; i < steps; i += 2) {
-    load(i + 1, r1);
-    __builtin_amdgcn_sched_barrier(0);
-    st_mul<MT, WK, CG>(r0, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    load(i + 2, r0);
-    __builtin_amdgcn_sched_barrier(0);
-    st_mul<MT, WK, CG>(r1, acc);
-    __builtin_amdgcn_sched_barrier(0);
+  int splits = p.splits;
+  for (;;) {
+    const int nblk = (ke - kb + 63) / 64;
+    const int steps = nblk > wb ? (nblk - wb + NWB - 1) / NWB * S : 0;
+    StStep<MT, WK, CG> r0, r1;
+    auto load = [&](int i, StStep<MT, WK, CG>& r) {
+      const int k = kb + 64 * (i / S * NWB + wb) + 32 * (i % S);
+      st_load<MT, WK, CG>(s, a, T, n0, k, i < steps && k < ke, lr, lg, r);
+    };
+    load(0, r0);
+    for (int i = 0; i < steps; i += 2) {
+      load(i + 1, r1);
+      __builtin_amdgcn_sched_barrier(0);
+      st_mul<MT, WK, CG>(r0, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      load(i + 2, r0);
+      __builtin_amdgcn_sched_barrier(0);
+      st_mul<MT, WK, CG>(r1, acc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" : "+s"(flag));  // not before the loop
+    if (splits == 1 || !flag) break;
+    if (split) return;
+    splits = 1;
+    kb = ke;
+    ke = s.K;
   }
+
+  const bool poison = flag != 0 && p.layer;
 
   // group g's column q of the tile (q = 8 lr + j)
   auto column = [&](int g, int q) { return CG == 1 ? q : (q >> 3) * (8 * CG) + 8 * g + (q & 7); };
@@ -268,6 +282,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(p.slices, 0, (int)p.slice_bytes, 0x00020000);
   const int gtile = blockIdx.y * p.tiles + tile;  // the tile's counter
   const uint32_t unit = (uint32_t)(gtile * p.splits + split) * BR;
+  const bool exchange = splits > 1 || p.out_t;
 #pragma unroll
   for (int g = 0; g < CG; ++g) {
     const int n = column(g, qn);
@@ -290,7 +305,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
         for (int w = 0; w < 8; ++w) v[w / NWB] += *reinterpret_cast<const f32x4*>(&red[w][qm * kStTileN + qn]);
         const int m = 16 * mt + qm;
         if (m < T && n0 + n < so.N) {
-          if (!p.exchange) {
+          if (!exchange) {
             store(m, n, finish(m, n, v[0], v[1]));
           } else {
 #pragma unroll
@@ -303,14 +318,14 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
       }
     }
   }
-  if (!p.exchange) return;
+  if (!exchange) return;
 
   // ---- K splits: the last unit of the tile to arrive sums the slices in
   // split order (the counter wraps to zero for the next launch) ----
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (tid == 0)
-    last = poison || p.splits == 1 ||
+    last = splits == 1 ||
            __builtin_amdgcn_atomic_inc32(dl_tile_counter(p.sync, gtile), (uint32_t)p.splits - 1u, __ATOMIC_RELAXED, "agent") ==
                (uint32_t)p.splits - 1u;
   __syncthreads();
@@ -323,14 +338,14 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
     const int g = CG == 1 ? 0 : q / (T * 32), m = (q >> 5) - g * T, n = column(g, 4 * (q & 31));
     if (n0 + n >= so.N) continue;
     f32x4 v[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    for (int s0 = 0; s0 < p.splits; s0 += SB) {
+    for (int s0 = 0; s0 < splits; s0 += SB) {
       u32x4 x[SB][BR];
 #pragma unroll
       for (int k = 0; k < SB; ++k)
 #pragma unroll
         for (int b = 0; b < BR; ++b)
           x[k][b] = __builtin_amdgcn_raw_buffer_load_b128(
-              rs, s0 + k < p.splits ? (unit0 + (uint32_t)((s0 + k) * BR + b)) * (srows * (uint32_t)(CG * kStTileN * 4)) + 16u * (uint32_t)q
+              rs, s0 + k < splits ? (unit0 + (uint32_t)((s0 + k) * BR + b)) * (srows * (uint32_t)(CG * kStTileN * 4)) + 16u * (uint32_t)q
                                     : kStNone,
               0, kDlSc1);
 #pragma unroll

@@ -107,7 +107,9 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
   __shared__ int last;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane & 15, lg = lane >> 4;
-  const bool poison = __hip_atomic_load(&p.sync[kDlFlag], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  // after a timeout on the workspace (its tile counters are in an unknown state)
+  // the first split's block takes its tile's whole K (stream.hpp)
+  uint64_t flag = p.sync[kDlFlag];
 
   // blocks in (split, column tile, row tile) order: the row tiles of a column
   // tile read the same weights
@@ -118,7 +120,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
   const StreamF32Seg& so = p.seg[second ? 1 : 0];
   const StreamF32Seg& s = p.seg[DUAL ? wave >> 2 : (second ? 1 : 0)];
   const int n0 = (second ? tile - p.seg[0].ntiles : tile) * kSfTileN;
-  const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
+  int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
 
   f32x4 acc[MT][4];
@@ -127,29 +129,37 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[mt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int nst = (ke - kb + 15) / 16;
-  const int steps = nst > wb ? (nst - wb + NWB - 1) / NWB : 0;
-  SfStep<MT> r0, r1;
-  auto load = [&](int i, SfStep<MT>& r) {
-    sf_load<MT, LIN, AT>(s, p.M, m0, n0, kb + 16 * (i * NWB + wb), i < steps, lr, lg, r);
-  };
-  load(0, r0);
-  for (int i = 0; i < steps; i += 2) {
-    load(i + 1, r1);
-    __builtin_amdgcn_sched_barrier(0);
-    sf_mul<MT, LIN>(r0, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    load(i + 2, r0);
-    __builtin_amdgcn_sched_barrier(0);
-    sf_mul<MT, LIN>(r1, acc);
-    __builtin_amdgcn_sched_barrier(0);
+  int splits = p.splits;
+  for (;;) {
+    const int nst = (ke - kb + 15) / 16;
+    const int steps = nst > wb ? (nst - wb + NWB - 1) / NWB : 0;
+    SfStep<MT> r0, r1;
+    auto load = [&](int i, SfStep<MT>& r) {
+      sf_load<MT, LIN, AT>(s, p.M, m0, n0, kb + 16 * (i * NWB + wb), i < steps, lr, lg, r);
+    };
+    load(0, r0);
+    for (int i = 0; i < steps; i += 2) {
+      load(i + 1, r1);
+      __builtin_amdgcn_sched_barrier(0);
+      sf_mul<MT, LIN>(r0, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      load(i + 2, r0);
+      __builtin_amdgcn_sched_barrier(0);
+      sf_mul<MT, LIN>(r1, acc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" : "+s"(flag));  // not before the loop
+    if (splits == 1 || !flag) break;
+    if (split) return;
+    splits = 1;
+    kb = ke;
+    ke = s.K;
   }
 
   auto finish = [&](int m, int n, f32x4 v0, f32x4 v1) {
     if constexpr (DUAL)
       v0 = f32x4{silu_f32(v0.x) * v1.x, silu_f32(v0.y) * v1.y, silu_f32(v0.z) * v1.z, silu_f32(v0.w) * v1.w};
     const int64_t off = (int64_t)m * so.N + n0 + n;
-    if (poison) v0 = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
     if (p.out_t) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) so.out[(int64_t)(n0 + n + i) * p.M + m] = v0[i];
@@ -179,7 +189,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
       for (int w = 0; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(&red[4 * half + w][qm * PITCH + qn]);
       const int m = m0 + 16 * mt + qm;
       const bool in = m < p.M && n0 + qn < so.N;
-      if (DUAL && p.splits > 1) {
+      if (DUAL && splits > 1) {
         if (in)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rs,
                                                  (((unit + half) * (16 * MT) + (16 * mt + qm)) * kSfTileN + qn) * 4u, 0, kDlSc1);
@@ -190,7 +200,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
         __syncthreads();
         if (!half && in) {
           const f32x4 o = hand[tid];
-          if (p.splits > 1)
+          if (splits > 1)
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v + o), rs,
                                                    ((unit * (16 * MT) + (16 * mt + qm)) * kSfTileN + qn) * 4u, 0, kDlSc1);
           else if (DUAL)
@@ -201,15 +211,15 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
       }
     }
   }
-  if (p.splits == 1) return;
+  if (splits == 1) return;
 
   // ---- K splits: the last block of the tile to arrive sums the slices in
   // split order ----
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (tid == 0)
-    last = poison || __builtin_amdgcn_atomic_inc32(dl_tile_counter(p.sync, t0), (uint32_t)p.splits - 1u, __ATOMIC_RELAXED,
-                                                   "agent") == (uint32_t)p.splits - 1u;
+    last = __builtin_amdgcn_atomic_inc32(dl_tile_counter(p.sync, t0), (uint32_t)splits - 1u, __ATOMIC_RELAXED, "agent") ==
+           (uint32_t)splits - 1u;
   __syncthreads();
   if (!last) return;
   const uint32_t unit0 = (uint32_t)(t0 * p.splits) * BR;
@@ -218,7 +228,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
     const int m = m0 + (q >> 4), n = 4 * (q & 15);
     if (m >= p.M || n0 + n >= so.N) continue;
     f32x4 v[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    for (int s0 = 0; s0 < p.splits; s0 += SB) {
+    for (int s0 = 0; s0 < splits; s0 += SB) {
       f32x4 x[SB][BR];
 #pragma unroll
       for (int k = 0; k < SB; ++k)
@@ -226,7 +236,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
         for (int b = 0; b < BR; ++b)
           x[k][b] = __builtin_bit_cast(
               f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                         rs, s0 + k < p.splits ? (unit0 + (uint32_t)((s0 + k) * BR + b)) * (16u * MT * kSfTileN * 4u) + 16u * (uint32_t)q
+                         rs, s0 + k < splits ? (unit0 + (uint32_t)((s0 + k) * BR + b)) * (16u * MT * kSfTileN * 4u) + 16u * (uint32_t)q
                                                : kStNone,
                          0, kDlSc1));
 #pragma unroll

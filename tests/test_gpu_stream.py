@@ -147,6 +147,53 @@ def test_stream_after_a_timeout(gpu):
     assert _rel(_np(ops.svd_mlp(xt, *ft, workspace=ws)), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
 
 
+def _flag_timeout(ws):
+    """The sync area as a timed-out persistent call may leave it."""
+    ws[2560:4096] = torch.arange(1536, device=ws.device).mul(37).remainder(251).to(torch.uint8)
+    ws[2304:2312].view(torch.int64).fill_(1)
+
+
+# The halves and fp32 calls have no waits: on a workspace whose timeout flag is
+# set, and whose tile counters hold anything, they compute as ever.  Stages
+# with K splits (d = 4160, fp8 in 256-column tiles among them) and without,
+# two row groups, the transposed result; fp32 from one token to several tiles.
+@pytest.mark.parametrize("T", [1, 16, 40, 72, 100])
+@pytest.mark.parametrize("kind", ["natural", "linear", "fp8"])
+def test_stream_halves_after_a_timeout(gpu, kind, T):
+    xb, wide, xt, ft = _layer(inputs.LayerShape(4160, 528, 136, 264), T, 30 + T, kind, gpu)
+    ops.clear_workspace_cache()
+    try:
+        h = ops.fused_gate_up(xt, *ft[:4])
+        ops.fused_xuv(h, *ft[4:])
+        for ws in ops._WS_CACHE.values():
+            _flag_timeout(ws)
+        h = ops.fused_gate_up(xt, *ft[:4])
+        assert _rel(_np(h), O.fused_gate_up_ref(xb, *wide[:4], dtype="bfloat16")) < TOL
+        y = ops.fused_xuv(h, *ft[4:])
+        assert _rel(_np(y), O.fused_xuv_ref(_np(h), *wide[4:], dtype="bfloat16")) < TOL
+        if T % 8 == 0:
+            assert torch.equal(ops.fused_gate_up(xt, *ft[:4], out_transposed=True).t(), h)
+        assert ops.workspace_status() is True
+    finally:
+        ops.clear_workspace_cache()
+
+
+@pytest.mark.parametrize("T", [1, 17, 128, 300])
+@pytest.mark.parametrize("kind", ["natural", "linear"])
+def test_f32_after_a_timeout(gpu, kind, T):
+    shape = inputs.LayerShape(1024, 3584, 256)
+    x, f = inputs.make_layer(shape, T=T, seed=600 + T)
+    xt, ft = torch.from_numpy(x).to(gpu), [torch.from_numpy(a).to(gpu) for a in f]
+    if kind == "linear":
+        ft = [a.t().contiguous().t() for a in ft]
+    ws = ops.svd_mlp_workspace(xt, r=shape.r, ff=shape.ff)
+    _flag_timeout(ws)
+    w = [a.double() for a in ft]
+    g = (xt.double() @ w[0]) @ w[1]
+    want = ((g * torch.sigmoid(g) * ((xt.double() @ w[2]) @ w[3])) @ w[4]) @ w[5]
+    assert float((ops.svd_mlp(xt, *ft, workspace=ws).double() - want).norm() / want.norm()) < 1e-5
+
+
 def test_fp8_transposed_odd_tokens_stay_refused(gpu):
     _, _, xt, ft = _layer(inputs.LayerShape(264, 528, 136), 9, 14, "fp8", gpu)
     for call in (lambda: ops.fused_gate_up(xt, *ft[:4], out_transposed=True),
