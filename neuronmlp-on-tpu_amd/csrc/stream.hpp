@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   // persistent layers do; the halves, which no wait precedes, run without the
   // counters: the first split's unit takes its tile's whole K.  The flag's load
   // is in flight with the weights' and looked at after them.
-  uint64_t flag = p.sync[kDlFlag];
+  const uint32_t flag = __hip_atomic_load(reinterpret_cast<uint32_t*>(&p.sync[kDlFlag]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   const int split = blockIdx.x / p.tiles;
   const int tile = blockIdx.x % p.tiles;
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const StreamSeg& so = p.seg[second ? 1 : 0];                        // the output's segment
   const StreamSeg& s = p.seg[DUAL ? wave >> 2 : (second ? 1 : 0)];  // the segment this wave streams
   const int n0 = (second ? tile - p.seg[0].ntiles : tile) * kStTileN * CG;
-  int kb = split * s.ks, ke = min(s.K, kb + s.ks);
+  const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
   const uint16_t* const a = s.a + (int64_t)m00 * s.K;
 
@@ -222,8 +222,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
 
   // step i of this wave: part i % S of its (i / S)-th 64-k block
   constexpr int S = 2 / StStep<MT, WK, CG>::H;
-  int splits = p.splits;
-  for (;;) {
+  auto run = [&](int kb, int ke) {
     const int nblk = (ke - kb + 63) / 64;
     const int steps = nblk > wb ? (nblk - wb + NWB - 1) / NWB * S : 0;
     StStep<MT, WK, CG> r0, r1;
@@ -242,12 +241,13 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
       st_mul<MT, WK, CG>(r1, acc);
       __builtin_amdgcn_sched_barrier(0);
     }
-    asm volatile("" : "+s"(flag));  // not before the loop
-    if (splits == 1 || !flag) break;
+  };
+  run(kb, ke);
+  int splits = p.splits;
+  if (splits > 1 && __builtin_amdgcn_readfirstlane(flag)) {
     if (split) return;
+    run(ke, s.K);
     splits = 1;
-    kb = ke;
-    ke = s.K;
   }
 
   const bool poison = flag != 0 && p.layer;

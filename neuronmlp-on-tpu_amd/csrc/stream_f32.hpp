@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
   const int lr = lane & 15, lg = lane >> 4;
   // after a timeout on the workspace (its tile counters are in an unknown state)
   // the first split's block takes its tile's whole K (stream.hpp)
-  uint64_t flag = p.sync[kDlFlag];
+  const uint32_t flag = __hip_atomic_load(reinterpret_cast<uint32_t*>(&p.sync[kDlFlag]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   // blocks in (split, column tile, row tile) order: the row tiles of a column
   // tile read the same weights
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
   const StreamF32Seg& so = p.seg[second ? 1 : 0];
   const StreamF32Seg& s = p.seg[DUAL ? wave >> 2 : (second ? 1 : 0)];
   const int n0 = (second ? tile - p.seg[0].ntiles : tile) * kSfTileN;
-  int kb = split * s.ks, ke = min(s.K, kb + s.ks);
+  const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
 
   f32x4 acc[MT][4];
@@ -129,8 +129,7 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[mt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  int splits = p.splits;
-  for (;;) {
+  auto run = [&](int kb, int ke) {
     const int nst = (ke - kb + 15) / 16;
     const int steps = nst > wb ? (nst - wb + NWB - 1) / NWB : 0;
     SfStep<MT> r0, r1;
@@ -148,12 +147,13 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
       sf_mul<MT, LIN>(r1, acc);
       __builtin_amdgcn_sched_barrier(0);
     }
-    asm volatile("" : "+s"(flag));  // not before the loop
-    if (splits == 1 || !flag) break;
+  };
+  run(kb, ke);
+  int splits = p.splits;
+  if (splits > 1 && __builtin_amdgcn_readfirstlane(flag)) {
     if (split) return;
+    run(ke, s.K);
     splits = 1;
-    kb = ke;
-    ke = s.K;
   }
 
   auto finish = [&](int m, int n, f32x4 v0, f32x4 v1) {
