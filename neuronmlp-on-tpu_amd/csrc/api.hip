@@ -21,7 +21,9 @@
 //   1-64 tokens, Linear-layout or fp8 factors, dimensions off the decode
 //   layer's tiles (multiples of 8), and the gate/up and x.u.v entry points;
 //   65-128 where the factors are small or off the large tiles (decode_ok):
-//                                    one streaming launch per stage (stream.hpp)
+//                                    one streaming launch per stage (stream.hpp),
+//                                    Linear-layout factors at 1-2 tokens a GEMV per
+//                                    stage (gemv_linear.hip)
 //   fp32, aligned:                   one fp32 streaming launch per stage
 //                                    (stream_f32.hpp)
 //   anything else (odd sizes):       the general 128x128 GEMM (gemm.hpp), whose
@@ -1474,6 +1476,7 @@ int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, boo
                          (int)K, (int)N[i], (int)((N[i] + bn - 1) / bn), ks};
   const char* why = nullptr;
   StageScope ss(stage, c.st);
+  if (w_lin && T <= kGlMaxT && !p.out_t) return check(launch_gemv_linear(p, nseg, dual, c.st, &why), what, why);
   return check(launch_stream(p, wk, cg, dual, c.st, &why), what, why);
 }
 

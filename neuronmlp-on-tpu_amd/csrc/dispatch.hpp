@@ -53,6 +53,8 @@ hipError_t launch_big(const BigDesc& d, const BigParams& p, int splits, int batc
 // columns (cg 2: fp8 up to 32 tokens), dual the gate/up pair of a column tile.
 struct StreamParams;
 hipError_t launch_stream(const StreamParams& p, int wk, int cg, bool dual, hipStream_t st, const char** why);
+// Linear-layout stage at one or two tokens (gemv_linear.hip) of `nseg` segments.
+hipError_t launch_gemv_linear(const StreamParams& p, int nseg, bool dual, hipStream_t st, const char** why);
 // fp32 streaming stage (stream_f32.hpp): mt 16-row token tiles a block, at:
 // activations given as (K, M).
 struct StreamF32Params;

@@ -78,6 +78,7 @@ struct StreamParams {
 constexpr int kStRows = 64;  // token rows of a group
 constexpr int kStMaxT = 2 * kStRows;
 constexpr int kStThreads = 512;
+constexpr int kGlMaxT = 2;  // tokens of the Linear GEMV stages (gemv_linear.hip)
 constexpr int kStTileN = 128;
 constexpr uint32_t kStNone = 0xfffffff0u;  // past the slice area: reads zeros
 

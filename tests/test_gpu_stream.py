@@ -71,6 +71,29 @@ def test_stream_entry_points(gpu, shape, kind, T):
         assert torch.equal(yT.view(torch.int16), y.view(torch.int16))
 
 
+# Linear factors at one and two tokens (csrc/gemv_linear.hip): K of one 8-wide
+# piece, short of and past one 512-k step, one batch of steps and two batches;
+# the block's residual; the same bits on replay and with a single token's row
+# in a call of two.
+@pytest.mark.parametrize("shape", [inputs.LayerShape(8, 16, 8), inputs.LayerShape(520, 1032, 504, 2056),
+                                   inputs.LayerShape(2048, 4104, 1160, 1032), inputs.LayerShape(4096, 8200, 72)])
+@pytest.mark.parametrize("T", [1, 2])
+def test_linear_gemv(gpu, shape, T):
+    xb, wide, xt, ft = _layer(shape, T, 60 + T, "linear", gpu)
+    h = ops.fused_gate_up(xt, *ft[:4])
+    assert _rel(_np(h), O.fused_gate_up_ref(xb, *wide[:4], dtype="bfloat16")) < TOL
+    y = ops.fused_xuv(h, *ft[4:])
+    assert _rel(_np(y), O.fused_xuv_ref(_np(h), *wide[4:], dtype="bfloat16")) < TOL
+    out = ops.svd_mlp(xt, *ft)
+    assert _rel(_np(out), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+    assert torch.equal(ops.svd_mlp(xt, *ft).view(torch.int16), out.view(torch.int16))
+    assert torch.equal(ops.svd_mlp(xt[:1].contiguous(), *ft).view(torch.int16), out[:1].view(torch.int16))
+    gain = torch.rand(shape.d, device=gpu) + 0.5
+    xn = (xt.float() * torch.rsqrt(xt.float().pow(2).mean(1, keepdim=True) + 1e-5) * gain).bfloat16()
+    want = (xt.float() + ops.svd_mlp(xn, *ft).float()).bfloat16()
+    assert _rel(_np(ops.svd_mlp_block(xt, gain, *ft)), _np(want)) < TOL
+
+
 # 65-128 tokens: a second group of token rows with units, slices and tile
 # counters of its own, from one row to full; K splits (d = 4160) and none,
 # dimensions that the large tiles take (512, 1024) and not, the transposed
