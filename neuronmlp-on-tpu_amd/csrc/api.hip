@@ -632,8 +632,11 @@ bool big_rank_ok(const Common& c, int64_t r) {
 }
 
 // Waves per block of a large-tile launch: 4 only for the fn-8 natural-layout
-// store stages under SVDMLP_TUNE=nw=4.
-int big_nw(int fn, int epi, bool b_kc) { return (fn == 8 && epi == BEPI_STORE && !b_kc && tune().nw == 4) ? 4 : 8; }
+// store stages under SVDMLP_TUNE=nw=4, and only of ranks in whole stages (the
+// rank maps' instances have 8).
+int big_nw(int fn, int epi, bool b_kc, bool mapped) {
+  return (fn == 8 && epi == BEPI_STORE && !b_kc && !mapped && tune().nw == 4) ? 4 : 8;
+}
 
 // Tile shapes whose fragment-order split-K slices the reduction kernel takes.
 bool big_frag_reduce_ok(int fn, int nw) { return (nw == 8 && fn >= 4 && fn <= 8 && fn != 5) || (nw == 4 && fn == 8); }
@@ -728,7 +731,7 @@ int big_gemm(const Common& c, int stage, const void* a0, const void* a1, int64_t
   }
   p.k_split = k_split;
   const int splits = (K + k_split - 1) / k_split;
-  const BigDesc d{fn, b_kc, epi, out_f32, fp8, kg == 2 ? 8 : big_nw(fn, epi, b_kc), kg};
+  const BigDesc d{fn, b_kc, epi, out_f32, fp8, kg == 2 ? 8 : big_nw(fn, epi, b_kc, nmap.shift || kmap.shift), kg};
   const char* why = nullptr;
   StageScope ss(stage, c.st);
   return check(launch_big(d, p, splits, batch, c.st, &why), "large-tile GEMM", why);
@@ -871,7 +874,7 @@ RankPlan plan_rank(int64_t T, int64_t K, int64_t N, int fn1, int batch, int64_t 
 // The split tail runs on the tile-range instance of the large-tile kernel:
 // 256 x 256 tiles of natural-layout bf16 B with 8 waves.
 bool xu_tail_ok(const Common& c, int fn, bool u_lin) {
-  return fn == 8 && c.wt == SVDMLP_BF16 && !u_lin && big_nw(fn, BEPI_STORE, u_lin) == 8;
+  return fn == 8 && c.wt == SVDMLP_BF16 && !u_lin && big_nw(fn, BEPI_STORE, u_lin, false) == 8;
 }
 
 // Split tail of the two-entry X.U stage (256-row tiles, fn * 32 wide): with
@@ -943,7 +946,7 @@ int big_xu2_tail(const Common& c, int stage, const void* a, int64_t lda, int64_t
                      part, r, 0, nullptr, true, sstride, s0, s1, 0, 1, &e1, nullptr, 1, 0, 0, head, rem)))
     return rc;
   const int splits = (K + tail_ks - 1) / tail_ks;
-  const int nw = big_nw(fn, BEPI_STORE, u_lin);
+  const int nw = big_nw(fn, BEPI_STORE, u_lin, false);
   StageScope fin(ST_FINALIZE, c.st);
   const int c0 = head / mt;  // first split column tile (both entries' tiles counted)
   if (c0 < nt0) {             // entry 0's split column tiles
@@ -963,7 +966,7 @@ int big_xu2(const Common& c, int stage, const void* a, int64_t lda, int64_t a_by
             int T, int K, int r, int r1, char* ws, const Ws& L, const float* const* su, int64_t ldu, int64_t ldu1) {
   const RankPlan pl = plan_rank(T, K, r, gate_xu_fn(T, K, r, 2, r1), 2, r1, !u_lin && c.wt == SVDMLP_BF16, stage);
   const int fn = pl.fn, kg = pl.kg;
-  const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, u_lin);
+  const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, u_lin, false);
   uint16_t* xu = reinterpret_cast<uint16_t*>(ws + L.xu_bf16);
   const int64_t ldb0 = u_lin ? K : (ldu ? ldu : r), ldb1 = u_lin ? K : (ldu1 ? ldu1 : r1);
   const int64_t b0 = (int64_t)(u_lin ? r : K) * ldb0 * wbytes(c), b1 = (int64_t)(u_lin ? r1 : K) * ldb1 * wbytes(c);
@@ -1051,7 +1054,7 @@ int big_xu(const Common& c, int stage, const void* a, int64_t lda, int64_t a_byt
                     BEPI_STORE, K, xu, r, (int64_t)T * r, nullptr, false, 0, s0, s1, 0, 0, nullptr, nullptr, kg, 0,
                     a_blk, 0, 0, nullptr, rk.map);
   float* part = reinterpret_cast<float*>(ws + L.part);
-  const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, u_lin);
+  const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, u_lin, rk.map.shift);
   if (kg == 2 || big_frag_reduce_ok(fn, nw)) {
     // slices in fragment order: per split, `batch` blocks of whole tiles
     const int64_t tp = (T + bm - 1) / bm * bm, np = ((int64_t)r + 32 * fn - 1) / (32 * fn) * (32 * fn), per = tp * np;
@@ -1224,7 +1227,7 @@ int big_swiglu(const Common& c, const uint16_t* xu_g, const uint16_t* xu_u, cons
     if (wrote_T) *wrote_T = tr;
     return check(launch_reduce_frag_bf16(upart, splits_u, per, per, static_cast<uint16_t*>(tr ? out_T : out), tr ? T : ff,
                                          (int64_t)T * ff, T, ff, mt, (int)(per / ((int64_t)bm * mt) / (32 * fn)), fn,
-                                         kg2 ? 8 : big_nw(fn, BEPI_STORE, v_lin), 1, c.st, fused ? nullptr : gbuf,
+                                         kg2 ? 8 : big_nw(fn, BEPI_STORE, v_lin, rk.map.shift), 1, c.st, fused ? nullptr : gbuf,
                                          nullptr, kg2 ? 2 : 1, fused ? part : nullptr, fused ? splits : 0, tr),
                  "split-K SwiGLU reduce");
   }
@@ -1390,7 +1393,7 @@ int big_v(const Common& c, const uint16_t* xu, const void* v, bool v_lin, int T,
                     rk.map);
   }
   float* part = reinterpret_cast<float*>(ws + L.part);
-  const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, v_lin);
+  const int nw = kg == 2 ? 8 : big_nw(fn, BEPI_STORE, v_lin, rk.map.shift);
   if (kg == 2 || big_frag_reduce_ok(fn, nw)) {
     if (c.blk) c.blk->resid_done = true;
     const int64_t tp = (T + bm - 1) / bm * bm, np = ((int64_t)dout + 32 * fn - 1) / (32 * fn) * (32 * fn), per = tp * np;

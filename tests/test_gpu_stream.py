@@ -426,3 +426,33 @@ def test_gate_values_keep_32_bits(gpu, kind, ff, r, T):
     h = ops.fused_gate_up(xt, *ft, out_transposed=True).t() if out_t else ops.fused_gate_up(xt, *ft)
     err = float((h.cpu().double() - want).norm())
     assert err < 1.05 * float((want.bfloat16().double() - want).norm())
+
+
+_NW4_CHILD = """
+import sys, numpy as np, torch
+sys.path[:0] = sys.argv[1].split("|")
+from svdmlp import fp8, inputs, ops
+x, f = inputs.make_layer(inputs.LayerShape(*map(int, sys.argv[2:6])), T=int(sys.argv[6]), seed=5)
+t = [inputs.to_torch(inputs.as_float32(a, torch.bfloat16), torch.bfloat16, torch.device("cuda:0")) for a in (x, *f)]
+if int(sys.argv[7]):
+    t = t[:1] + [fp8.quantize_per_channel(a) for a in t[1:]]
+np.save(sys.argv[8], ops.svd_mlp(*t).view(torch.int16).cpu().numpy())
+"""
+
+
+# The 4-wave tiles (SVDMLP_TUNE=nw=4) have no rank-map instance: such ranks run
+# with 8 waves, to the bits of the default.  kg=0: 256-row tiles everywhere, so
+# that the 256-wide store stages are reached.
+@pytest.mark.parametrize("q", [0, 1])
+def test_ranks_off_the_stages_with_four_wave_tiles(gpu, tmp_path, q):
+    import os
+    import subprocess
+    import sys
+
+    got = []
+    for tune in ("nw=4,kg=0", "kg=0"):
+        out = tmp_path / f"{tune}.npy"
+        subprocess.run([sys.executable, "-c", _NW4_CHILD, "|".join(p for p in sys.path if p), "1024", "2048", "1136", "496",
+                        "600", str(q), str(out)], env=dict(os.environ, SVDMLP_TUNE=tune), check=True, timeout=120)
+        got.append(np.load(out))
+    assert np.array_equal(*got)
