@@ -79,8 +79,8 @@ extern "C" {
  * would exceed the 3e-2 fp8 tolerance (LLaMA3-70B shape: the layer with the
  * flag is ~2.7% from the math on dequantised factors, against 0.5% without).
  * Taken on the large-tile path (more than 64 tokens) where ff is a multiple
- * of 128 and r_d of 16; other shapes run as without it.  bf16 factors:
- * SVDMLP_EINVAL. */
+ * of 128 and d and the ranks of 32; other shapes run as without it.  bf16
+ * factors: SVDMLP_EINVAL. */
 #define SVDMLP_FP8_ACT 0x20u
 
 /* status codes */

@@ -2452,7 +2452,7 @@ int svd_mlp_run(const void* x, const void* ug, const void* vg, const void* uu, c
     const uint16_t* xu = reinterpret_cast<const uint16_t*>(ws + L.xu_bf16);
     uint16_t* hbuf = reinterpret_cast<uint16_t*>(ws + L.h);
     uint16_t* gbuf = reinterpret_cast<uint16_t*>(ws + L.g);
-    const bool f8a = fp8_act && r_d % 32 == 0 && f8_down_ok(T, ff, r_d, ld.ud);
+    const bool f8a = fp8_act && r_gu % 32 == 0 && r_d % 32 == 0 && f8_down_ok(T, ff, r_d, ld.ud);
     bool hblk = !f8a && tune().hblk;
     if ((rc = big_swiglu(c, xu, xu + T * big_rank(r_gu).p, vg, vu, v_lin, T, r_gu, ff, gbuf, hbuf,
                          reinterpret_cast<float*>(ws + L.part), (int64_t)(L.norm - L.part), S[1], S[3], ld.v, 0, 0,

@@ -328,6 +328,18 @@ def test_ranks_off_the_stages(gpu, shape, kind, T):
         assert _rel(_np(blk), _np((xt.float() + ops.svd_mlp(xn, *ft).float()).bfloat16())) < TOL
 
 
+# e4m3 h (SVDMLP_FP8_ACT) is for ranks in whole 32-k stages: with the gate/up
+# or the down rank off them the layer runs as without the flag, to its bits.
+@pytest.mark.parametrize("T", [65, 128, 300])
+@pytest.mark.parametrize("shape", [inputs.LayerShape(512, 1024, 336, 256), inputs.LayerShape(512, 1024, 256, 336)])
+def test_ranks_off_the_stages_keep_bf16_h(gpu, shape, T):
+    xb, wide, xt, ft = _layer(shape, T, 40 + T, "fp8", gpu)
+    got = ops.svd_mlp(xt, *ft, fp8_activations=True)
+    assert _rel(_np(got), O.svd_mlp_ref(xb, *wide, dtype="bfloat16")) < TOL
+    if T > 128:  # (below, the flag keeps the large tiles where the streaming stages are the default)
+        assert torch.equal(got.view(torch.int16), ops.svd_mlp(xt, *ft).view(torch.int16))
+
+
 # An infinite weight among the rows that the last 64-rank block repeats gives
 # infinities by the sign of its rank value, not NaN (infinity times zero).
 @pytest.mark.parametrize("T", [65, 300, 1030])
