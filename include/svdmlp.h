@@ -99,7 +99,12 @@ const char* svdmlp_last_error(void);
  * Workspace bytes needed by svdmlp_gate_up, svdmlp_xuv and svdmlp_svd_mlp for
  * T tokens, hidden size d, intermediate size ff and (maximum) rank r.  The
  * same workspace may be reused by consecutive calls on one stream of one
- * device.  Its first 4096 bytes must be zero before its first use: they hold
+ * device.  The size is not monotone in T: a workspace for several token counts
+ * takes the largest of theirs.  A smaller one that still holds what every call
+ * needs is accepted; its calls at up to 4 tokens then run without the
+ * contracted layer's area, those of the streaming stages at up to 32 with
+ * fewer K splits (slower, and other last bits).  A workspace for more than 32
+ * tokens holds the streaming stages' area for any fewer.  Its first 4096 bytes must be zero before its first use: they hold
  * the grid-barrier and block-done counters of the persistent decode kernels
  * (the streaming-GEMV layer at 1-2 tokens and the MFMA layer up to 128),
  * which only ever grow, and the MFMA layer's split-K tile counters (from byte
@@ -240,7 +245,8 @@ int svdmlp_svd_mlp_block_ranks(const void* x, const float* norm_w, float eps, co
  * nothing.  No counterpart in the reference; it is for callers that cannot
  * allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Shapes whose workspace
- * (svdmlp_workspace_bytes) exceeds 64 MiB are rejected with SVDMLP_EINVAL
+ * (svdmlp_workspace_bytes, less the areas at its end that a call can do
+ * without) exceeds 64 MiB are rejected with SVDMLP_EINVAL
  * (LLaMA3-8B: up to 64 tokens; prefill shapes need a workspace).  The first
  * call on a device looks the scratch up and clears its sync area on `stream`
  * (the current device's).  Every call on a device shares that device's

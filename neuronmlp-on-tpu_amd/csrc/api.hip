@@ -186,6 +186,9 @@ constexpr int64_t kDlContractMaxT = 4;
 constexpr int64_t kDlContractAutoPadded = 2;
 constexpr int64_t kDlContractAutoDense = 3;
 
+// Tokens up to which the streaming stages' slices have an area of their own.
+constexpr int64_t kStreamXT = 32;
+
 struct Ws {
   size_t sync;     // 4 KB of grid-barrier words (zero before first use)
   size_t xu_bf16;  // [2][T][r] bf16 (gate, up) rank-r intermediate
@@ -200,7 +203,7 @@ struct Ws {
   size_t need;     // bytes every call needs (the regions above)
   size_t cslices;  // partial XU_d tiles of the contracted decode layer (T <= kDlContractMaxT), last: a
                    // workspace without them runs the other decode layers
-  size_t xslices;  // slices of the streaming stages at up to 32 tokens, last: without them they use `slices`
+  size_t xslices;  // slices of the streaming stages at up to kStreamXT tokens, last: without them they use `slices`
   size_t total;
 };
 
@@ -299,11 +302,12 @@ Ws ws_layout(int64_t T, int64_t d, int64_t ff, int64_t r) {
              ? a256(dl_contract_bytes(r / 128, ff / 64, T))
              : 0;
   // the streaming stages' slices where `slices` is short of them: 256 units
-  // of two branches and 256 columns, T rows each (kDecodeMaxT tokens with 128
-  // columns fit `slices`)
+  // of two branches and 256 columns, T rows each (33 tokens and more, with 128
+  // columns, fit `slices`).  A workspace for more tokens is as large as one for
+  // kStreamXT, so that fewer tokens have the same K splits in either.
   w.xslices = off;
-  off += T <= 32 ? a256(T * 1024 * 128 * 4) : 0;
-  w.total = off;
+  off += T <= kStreamXT ? a256(T * 1024 * 128 * 4) : 0;
+  w.total = T <= kStreamXT ? off : std::max(off, ws_layout(kStreamXT, d, ff, r).total);
   return w;
 }
 
@@ -1446,8 +1450,8 @@ int stream_splits(int64_t K, int64_t tiles, int64_t slice, int64_t area, int* ks
   return (int)((K + *ks - 1) / *ks);
 }
 
-int64_t stream_area(const Ws& L, size_t ws_bytes, size_t* off) {
-  const bool x = ws_bytes >= L.total && L.total > L.xslices;  // the larger area at the end
+int64_t stream_area(int64_t T, const Ws& L, size_t ws_bytes, size_t* off) {
+  const bool x = T <= kStreamXT && ws_bytes >= L.total;  // the larger area at the end
   *off = x ? L.xslices : L.slices;
   return std::min<int64_t>((int64_t)(x ? L.total - L.xslices : L.need - L.slices), 0x7ffffff0);
 }
@@ -1466,7 +1470,7 @@ int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, boo
   for (int i = 0; i < nseg; ++i) p.tiles += !dual || i == 0 ? (int)((N[i] + bn - 1) / bn) : 0;
   p.groups = (int)((T + kStRows - 1) / kStRows);
   size_t off = 0;
-  const int64_t area = stream_area(L, ws_bytes, &off);
+  const int64_t area = stream_area(T, L, ws_bytes, &off);
   p.slices = reinterpret_cast<float*>(ws + off);
   p.slice_bytes = (uint32_t)area;
   p.splits = stream_splits(K, p.groups * p.tiles, (dual ? 2 : 1) * std::min<int64_t>(T, kStRows) * bn * 4, area, &ks);
@@ -1488,7 +1492,7 @@ int stream_stage(const Common& c, int stage, int64_t T, int64_t K, int nseg, boo
 bool stream_out_t_ok(int64_t T, int64_t N, const Ws& L, size_t ws_bytes) {
   const int64_t tiles = (N + 2 * kStTileN - 1) / (2 * kStTileN) * 2 * ((T + kStRows - 1) / kStRows);
   size_t off = 0;
-  return tiles <= kDlMaxTiles && tiles * 2 * std::min<int64_t>(T, kStRows) * kStTileN * 4 <= stream_area(L, ws_bytes, &off);
+  return tiles <= kDlMaxTiles && tiles * 2 * std::min<int64_t>(T, kStRows) * kStTileN * 4 <= stream_area(T, L, ws_bytes, &off);
 }
 
 // Streaming stages take bf16 activations and any bf16 or fp8 factors in rows

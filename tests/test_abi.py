@@ -57,6 +57,14 @@ def test_version_and_workspace(lib):
         assert lib.svdmlp_workspace_bytes(T, 4096, 14336, 2816, 1) >= 22 * 224 * T * 512
 
 
+def test_a_workspace_for_more_tokens_holds_fewer(lib):
+    # the streaming stages' slice area at up to 32 tokens is in every larger workspace
+    for dims in ((4096, 14336, 2816), (3072, 8192, 1792), (1024, 3584, 256), (256, 512, 128), (8, 8, 8)):
+        few = max(lib.svdmlp_workspace_bytes(T, *dims, 1) for T in range(5, 33))
+        for T in (33, 40, 64, 65, 128, 129, 200, 513, 2048):
+            assert lib.svdmlp_workspace_bytes(T, *dims, 1) >= few, (dims, T)
+
+
 def _call_gate_up(lib, T=4, d=16, ff=32, r=8, act=1, wt=1, flags=0, ptr=256, ws=1 << 20):
     p = ctypes.c_void_p(ptr)
     return lib.svdmlp_gate_up(p, p, p, p, p, None, None, None, None, p, T, d, ff, r, act, wt, flags,

@@ -158,6 +158,19 @@ def test_stream_small_workspace(gpu):
         assert _rel(_np(ops.svd_mlp(xt, *ft, workspace=w)), want) < TOL
 
 
+@pytest.mark.parametrize("kind", ["linear", "fp8"])
+def test_stream_workspace_of_more_tokens(gpu, kind):
+    """The bits do not depend on which larger token count the workspace is for."""
+    shape = inputs.LayerShape(2048, 8192, 1792)
+    xb, wide, xt, ft = _layer(shape, 30, 17, kind, gpu)
+    code = _lib.SVDMLP_FP8_E4M3 if kind == "fp8" else _lib.SVDMLP_BF16
+    want = ops.svd_mlp(xt, *ft, workspace=ops.svd_mlp_workspace(xt, r=shape.r, ff=shape.ff, w_code=code))
+    for T in (33, 64, 65):
+        more = torch.empty(T, shape.d, dtype=xt.dtype, device=gpu)
+        ws = ops.svd_mlp_workspace(more, r=shape.r, ff=shape.ff, w_code=code)
+        assert torch.equal(ops.svd_mlp(xt, *ft, workspace=ws).view(torch.int16), want.view(torch.int16)), T
+
+
 def test_stream_after_a_timeout(gpu):
     """A workspace whose timeout flag is set gives NaN until it is reset (the
     tile counters may hold anything then)."""
