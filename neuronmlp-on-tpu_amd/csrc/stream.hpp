@@ -34,8 +34,8 @@
 // Measured (rotating weights, against the kernels before this one: register
 // loads of a whole slice and then its MFMAs, software fp8 widening, LDS and
 // global float atomics, zero-fill and conversion passes): 70B fp8 layer at 4
-// tokens 800 -> 130 us (623 MB; its XU.V stage streams 323 MB in 61 us, 5.3
-// TB/s), 8B Linear-layout layer at 16 tokens 170 -> 82 us, 8B x.u.v at 32
+// tokens 800 -> 130 us (623 MB; its XU.V stage streams 323 MB in 61.0 us on
+// average, 5.3 TB/s, reading 1.01 times its factors), 8B Linear-layout layer at 16 tokens 170 -> 82 us, 8B x.u.v at 32
 // tokens 114 -> 33 us.  What is left per launch is ~3.5-4.5 us of launch,
 // ramp and in-block sums and 1.5 us (16 tokens) to 4 us (64) of slices.
 // At 65-128 tokens two groups of 64 rows run side by side as blocks of their
@@ -196,13 +196,8 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const int m00 = blockIdx.y * kStRows;     // the group's first token row
   const int T = min(p.T - m00, kStRows);    // and its rows
   const uint32_t srows = min(p.T, kStRows);  // rows of a slice
-  // A workspace whose persistent decode call timed out has tile counters in an
-  // unknown state.  The layer then gives NaN until it is reset, as the
-  // persistent layers do; the halves, which no wait precedes, run without the
-  // counters: the first split's unit takes its tile's whole K.  The flag's load
-  // is in flight with the weights' and looked at after them.
-  const uint32_t flag = __hip_atomic_load(reinterpret_cast<uint32_t*>(&p.sync[kDlFlag]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-
+  int splits = p.splits;
+  asm volatile("" : "+s"(splits));  // loaded with the arguments above, not after the weights
   const int split = blockIdx.x / p.tiles;
   const int tile = blockIdx.x % p.tiles;
   const bool second = !DUAL && tile >= p.seg[0].ntiles;
@@ -212,6 +207,13 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
   const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
   const uint16_t* const a = s.a + (int64_t)m00 * s.K;
+
+  // A workspace whose persistent decode call timed out has tile counters in an
+  // unknown state.  The layer then gives NaN until it is reset, as the
+  // persistent layers do; the halves, which no wait precedes, run without the
+  // counters: the first split's unit takes its tile's whole K.  The flag's load
+  // is in flight with the weights' and looked at after them.
+  const uint32_t flag = __hip_atomic_load(reinterpret_cast<uint32_t*>(&p.sync[kDlFlag]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   f32x4 acc[CG][MT][8];
 #pragma unroll
@@ -244,7 +246,6 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_kernel(StreamParams p) {
     }
   };
   run(kb, ke);
-  int splits = p.splits;
   if (splits > 1 && __builtin_amdgcn_readfirstlane(flag)) {
     if (split) return;
     run(ke, s.K);

@@ -107,21 +107,24 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
   __shared__ int last;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane & 15, lg = lane >> 4;
-  // after a timeout on the workspace (its tile counters are in an unknown state)
-  // the first split's block takes its tile's whole K (stream.hpp)
-  const uint32_t flag = __hip_atomic_load(reinterpret_cast<uint32_t*>(&p.sync[kDlFlag]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int splits = p.splits, nt0 = p.seg[0].ntiles;
+  asm volatile("" : "+s"(splits), "+s"(nt0));  // loaded with the other arguments, not on their own later
 
   // blocks in (split, column tile, row tile) order: the row tiles of a column
   // tile read the same weights
   const int all = p.tiles * p.mtiles;
   const int split = blockIdx.x / all, t0 = blockIdx.x % all;
   const int tile = t0 / p.mtiles, m0 = t0 % p.mtiles * (16 * MT);
-  const bool second = !DUAL && tile >= p.seg[0].ntiles;
+  const bool second = !DUAL && tile >= nt0;
   const StreamF32Seg& so = p.seg[second ? 1 : 0];
   const StreamF32Seg& s = p.seg[DUAL ? wave >> 2 : (second ? 1 : 0)];
-  const int n0 = (second ? tile - p.seg[0].ntiles : tile) * kSfTileN;
+  const int n0 = (second ? tile - nt0 : tile) * kSfTileN;
   const int kb = split * s.ks, ke = min(s.K, kb + s.ks);
   const int wb = DUAL ? wave & 3 : wave;
+
+  // after a timeout on the workspace (its tile counters are in an unknown state)
+  // the first split's block takes its tile's whole K (stream.hpp)
+  const uint32_t flag = __hip_atomic_load(reinterpret_cast<uint32_t*>(&p.sync[kDlFlag]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   f32x4 acc[MT][4];
 #pragma unroll
@@ -149,7 +152,6 @@ __global__ __launch_bounds__(kStThreads, 2) void stream_f32_kernel(StreamF32Para
     }
   };
   run(kb, ke);
-  int splits = p.splits;
   if (splits > 1 && __builtin_amdgcn_readfirstlane(flag)) {
     if (split) return;
     run(ke, s.K);
