@@ -26,9 +26,9 @@
  *   - Return value: 0 on success; SVDMLP_EINVAL for an invalid argument (the
  *     message is available from svdmlp_last_error(), thread-local); SVDMLP_EHIP
  *     for a HIP runtime error.
- *   - Decode shapes (1 to 128 tokens, bf16) run as one persistent launch of
- *     one block per CU whose phases meet at grid barriers; it needs the whole
- *     device.  Do not run it concurrently with other work on the device
+ *   - Layer calls at decode shapes (1 to 128 tokens, bf16 natural-layout
+ *     factors) run as one persistent launch of one block per CU whose phases
+ *     meet at grid barriers; it needs the whole device.  Do not run it concurrently with other work on the device
  *     (another stream, another process): blocks that cannot become resident
  *     stall the barriers, whose bounded waits then give up.  A call whose
  *     wait gave up writes NaN into y wherever the result could be incomplete
@@ -107,9 +107,12 @@ const char* svdmlp_last_error(void);
  * tokens holds the streaming stages' area for any fewer.  Its first 4096 bytes must be zero before its first use: they hold
  * the grid-barrier and block-done counters of the persistent decode kernels
  * (the streaming-GEMV layer at 1-2 tokens and the MFMA layer up to 128),
- * which only ever grow, and the MFMA layer's split-K tile counters (from byte
- * 2560), which every call leaves at zero.  The 64-bit word at byte 2304 is
- * the timeout flag (see svdmlp_workspace_status); a nonzero 32-bit value at
+ * which only ever grow, and the split-K tile counters (from byte 2560) of the
+ * MFMA layer and of the streaming stages, which every call leaves at zero.
+ * The streaming stages are what gate/up, x.u.v, fp8, Linear-layout and
+ * off-tile layer calls at up to 128 tokens run, and aligned fp32 calls at any
+ * token count, so the rule holds for every entry point.  The 64-bit word at
+ * byte 2304 is the timeout flag (see svdmlp_workspace_status); a nonzero 32-bit value at
  * byte 2312 replaces the default bound of the barrier waits (in polls of
  * about a microsecond; failure tests set a tiny one).
  * Replaces the VMEM planning of test_speedup.py:208-258 (the TPU kernels keep
@@ -122,8 +125,11 @@ size_t svdmlp_workspace_bytes(int64_t T, int64_t d, int64_t ff, int64_t r, int32
  * in the reference, whose kernels have no cross-block waits).  Returns 1 if a
  * grid-barrier wait of an earlier call on this workspace gave up (those calls
  * wrote NaN into y wherever their result could be incomplete; the flag stays
- * set, and later decode calls write NaN too, until reset), 0 if none did, or a
- * negative status.  Waits for `stream` (a hipStream_t) first.  With reset
+ * set until reset), 0 if none did, or a negative status.  While it is set,
+ * svdmlp_svd_mlp* calls that run the persistent layers, or the bf16 and fp8
+ * streaming stages at up to 128 tokens, write NaN too; svdmlp_gate_up,
+ * svdmlp_xuv, fp32, large-tile and Linear-layout calls at one or two tokens
+ * compute as ever.  Waits for `stream` (a hipStream_t) first.  With reset
  * nonzero it then zeroes the 4096-byte sync area (stream-ordered), which makes
  * the workspace usable again; no call may be in flight on the workspace then.
  * The reference rejects non-finite layer outputs (test_speedup.py:852-853,
@@ -174,9 +180,10 @@ int svdmlp_svd_mlp(const void* x, const void* ug, const void* vg, const void* uu
  * models/modeling_llama.py:253-262.  The persistent decode layers run the
  * whole block in their one launch (a phase 0 writes RMSNorm(x), one block
  * per token row, before the layer's first grid barrier; the last phase adds
- * the residual as it writes y); the streaming-GEMV layer and the large-tile
- * path add the residual in their output stage after a separate RMSNorm pass;
- * the other paths run both as passes of their own.
+ * the residual as it writes y); the streaming-GEMV layer, the streaming
+ * stages (fp32 ones too) and the large-tile path add the residual in their
+ * output stage after a separate RMSNorm pass; unaligned calls run both as
+ * passes of their own.
  */
 int svdmlp_svd_mlp_block(const void* x, const float* norm_w, float eps, const void* ug, const void* vg,
                          const void* uu, const void* vu, const void* ud, const void* vd,

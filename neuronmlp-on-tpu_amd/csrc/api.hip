@@ -192,14 +192,14 @@ constexpr int64_t kStreamXT = 32;
 struct Ws {
   size_t sync;     // 4 KB of grid-barrier words (zero before first use)
   size_t xu_bf16;  // [2][T][r] bf16 (gate, up) rank-r intermediate
-  size_t xu32;     // [3][T][r] fp32 (gate, up, down) split-K accumulators
-  size_t gu32;     // [2][T][big] fp32 gate/up sums (decode)
+  size_t xu32;     // [3][T][r] fp32 XU (gate, up, down): fp32 stages, GEMV layer and general GEMM
+  size_t gu32;     // [2][T][big] fp32 gate/up sums of the streaming-GEMV layer, bf16 XU_d of the MFMA decode layer
   size_t h;        // [T][big] h of the fused layer (4 bytes/elem worst case)
-  size_t y32;      // [T][big] fp32 output accumulator (decode)
+  size_t y32;      // [T][big] fp32 output sums of the streaming-GEMV layer, fp32 stages' slices above kDlMaxT tokens
   size_t part;     // [splits][batch][T][N] fp32 split-K partial slices (prefill)
   size_t norm;     // [T][d] RMSNorm output of the MLP block (4 bytes/elem worst case)
   size_t g;        // bf16 gate values of the large-tile g pass, fragment order over padded tiles
-  size_t slices;   // split-K partial sums of the MFMA decode layer (decode only)
+  size_t slices;   // split-K partial sums of the MFMA decode layer and the streaming stages (up to kDlMaxT tokens)
   size_t need;     // bytes every call needs (the regions above)
   size_t cslices;  // partial XU_d tiles of the contracted decode layer (T <= kDlContractMaxT), last: a
                    // workspace without them runs the other decode layers
@@ -1510,6 +1510,11 @@ bool stream_out_t_ok(int64_t T, int64_t N, const Ws& L, size_t ws_bytes) {
 // 97, (2048, 5632, 1152) 95 / 91 -> 70 / 73; at 104 MB (8B) 153 / 158 -> 172 /
 // 183.  Natural bf16 stays on the K-group tiles: (3072, 8192, 1736) 81 / 82 us
 // there, 80 / 89 streamed (smaller layers gain a little, 17 MB 68 / 66 -> 62 / 64).
+// Nearer the lines, T=65 / 96 / 128: fp8 (5120, 13824, 3264), 62 MB, 167 / 163 /
+// 164 -> 121 / 128 / 139; Linear (3584, 9472, 1792), 47 MB, 128 / 124 / 124 ->
+// 111 / 113 / 119.  Past them the token count decides: fp8 92 MB 192 / 193 / 196
+// -> 139 / 151 / 167, 131 MB 256 / 257 / 262 -> 221 / 239 / 276; Linear 50 MB
+// 121 / 120 / 118 -> 112 / 114 / 121, 75 MB 135 / 134 / 134 -> 124 / 126 / 133.
 bool decode_ok(const Common& c, int64_t T, std::initializer_list<int64_t> dims, bool vec, bool lin, int64_t pair, bool big) {
   if (c.f32 || !vec || T > kStMaxT) return false;
   const bool f8 = c.wt == SVDMLP_FP8_E4M3;
@@ -1612,9 +1617,12 @@ int f32_xuv(const Common& c, const void* a, const void* u, const void* v, bool u
 // The persistent decode layer takes bf16 activations and factors in natural
 // layout, T <= kDlMaxT, ranks and d multiples of 128 and ff a multiple of 64
 // (its tiles), every operand below 2 GB (32-bit buffer offsets).
-// It beats the per-stage decode kernels at every T (measured on MI355X, 8B
-// shape: T=1 83 us vs 88 us; T=8 82 vs 95; T=64 118 vs 250); the
-// streaming-GEMV layer, tried first, takes 1 <= T <= kGvMaxT.
+// Against the streaming stages (SVDMLP_TUNE=dlayer=0,gvmax=0; dense factors,
+// us per layer, this one / the stages): 8B T=1 / 8 / 16 / 32 / 64 / 128 70.0 /
+// 74.7 / 76.7 / 76.8 / 86.4 / 115.5 against 70.8 / 72.8 / 76.0 / 87.2 / 110 /
+// 123; (3072, 8192, 1792) T=8 / 32 / 128 43.5 / 48.0 / 67.7 against 42.2 / 53.1
+// / 82.9.  Up to 16 tokens the stages are level at these sizes and faster on
+// small layers ((1024, 3584, 256) T=16 33.7 against 24.2), which no rule uses yet.
 constexpr int64_t kDlMinT = 1;
 
 // r_u: the up branch's rank (r_gu the gate's); with distinct ranks phase 2

@@ -84,7 +84,6 @@ struct GvParams;
 int gemv_layer_grid(int rw);
 int gemv_layer_a_floats();
 hipError_t launch_gemv_layer(const GvParams& p, int rw, int grid, hipStream_t st, const char** why);
-hipError_t launch_cvt_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t st);
 // out[i] = bf16(sum_s in[s * stride + i]) for s < slices.
 hipError_t launch_reduce_bf16(const float* in, int slices, int64_t stride, uint16_t* out, int64_t n,
                               hipStream_t st);
@@ -94,8 +93,8 @@ hipError_t launch_reduce_bf16(const float* in, int slices, int64_t stride, uint1
 // (kg 2, nw 8: four wave tiles), batch entries zb (out batch stride
 // obstride elements); with `gate` (bf16 in the same fragment order),
 // out = bf16(SiLU(gate) * sum); with `gsl` (gsplits fp32 slices of the gate
-// in the same layout and slice stride), the gate is bf16(sum of its slices
-// in order) first, as launch_reduce_bf16 would round it; with `resid` (bf16,
+// in the same layout and slice stride), the gate is the sum of its slices in
+// order, in 32 bits; with `resid` (bf16,
 // row pitch ldo, batch entry 0), out = bf16(resid + bf16(sum)), the MLP
 // block's residual add; with out_t out is (N, M), M a multiple of 8.
 hipError_t launch_reduce_frag_bf16(const float* in, int splits, int64_t sstride, int64_t bstride, uint16_t* out,

@@ -1,4 +1,4 @@
-// Small elementwise kernels: zero fill, fp32 -> bf16, split-K slice sums.
+// Small elementwise kernels: zero fill, split-K slice sums.
 #include "dispatch.hpp"
 
 namespace svdmlp {
@@ -12,28 +12,6 @@ __global__ void fill_zero_kernel(float* p, int64_t n) {
       for (int64_t t = i; t < n; ++t) p[t] = 0.0f;
     }
   }
-}
-
-// out[i] = bf16(in[i]), eight elements per thread and step.
-__global__ void cvt_bf16_kernel(const float* in, uint16_t* out, int64_t n) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x * 8;
-  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8; i < n; i += stride) {
-    if (i + 7 < n) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(in + i);
-      const f32x4 b = *reinterpret_cast<const f32x4*>(in + i + 4);
-      *reinterpret_cast<u32x4*>(out + i) = u32x4{pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w),
-                                                 pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w)};
-    } else {
-      for (int64_t t = i; t < n; ++t) out[t] = (uint16_t)f32_to_bf16_bits(in[t]);
-    }
-  }
-}
-
-hipError_t launch_cvt_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  const int blocks = (int)std::min<int64_t>((n / 8 + 255) / 256 + 1, 2048);
-  hipLaunchKernelGGL(cvt_bf16_kernel, dim3(blocks), dim3(256), 0, st, in, out, n);
-  return hipGetLastError();
 }
 
 // out[i] = bf16(sum over split-K slices), eight elements per thread and step;

@@ -291,6 +291,24 @@ def test_f32_stages(gpu, shape, kind, T):
     assert rel(ops.svd_mlp_block(xt, gain, *ft), want) < 1e-5
 
 
+# SiLU over the range of its exponential.  U and V are identities, so the gate
+# and the up value are x itself.  For x < 0 exp(-x) carries the rounding of its
+# argument, |x| 2^-24 relative and as much again for the log2(e) it is
+# multiplied with, and 1 + exp(-x), the reciprocal and the two products a unit
+# in the last place each; from about -87.3 on the reciprocal would be
+# subnormal and the result is zero, |x| 2^-126 off at most.
+@pytest.mark.parametrize("T", [3, 200])
+def test_silu_over_the_range_of_its_exponential(gpu, T):
+    d = 256
+    x = torch.linspace(-110, 110, T * d, device=gpu, dtype=torch.float64).float().reshape(T, d)
+    eye = torch.eye(d, device=gpu)
+    got = ops.fused_gate_up(x, eye, eye, eye, eye).double()
+    x = x.double()
+    want = x * torch.sigmoid(x) * x
+    bound = want.abs() * (2 * x.abs() + 16) * 2.0**-24 + x * x * 2.0**-126
+    assert ((got - want).abs() <= bound).all()
+
+
 # The persistent decode layer's phase 2 in K splits (layers narrower than the
 # grid): 2 (3B-like ratio) and 9 (ff = 1792, rank 2304) ways, distinct gate and
 # up ranks whose splits end apart, the last-arrival (up to 16 tokens) and the

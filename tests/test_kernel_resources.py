@@ -38,7 +38,7 @@ def test_report_covers_the_kernels():
     rep = _report()
     names = set(rep)
     for frag in ("big_gemm_kernel", "f8_gemm_kernel", "decode_layer_kernel", "gemv_layer_kernel",
-                 "reduce_frag_bf16_kernel"):
+                 "reduce_frag_bf16_kernel", "stream_kernel", "stream_f32_kernel", "gemv_linear_kernel"):
         assert any(frag in n for n in names), frag
     for n, r in rep.items():
         assert {"VGPRs", "AGPRs", "ScratchSize [bytes/lane]", "VGPRs Spill"} <= set(r), n
