@@ -180,8 +180,7 @@ size_t a256(int64_t x) { return ((size_t)x + 255) & ~(size_t)255; }
 // 66.54 vs 65.47, T=3 66.69 vs 67.44, T=4 67.02 vs 69.10), with dense factors
 // up to three (the four-phase layer with one-branch phase-2 units against
 // contracted: T=1 72.47 vs 71.05, T=2 71.77 vs 71.04, T=3 73.32 vs 72.82, T=4
-// 73.40 vs 74.78; before this round's decode changes the four-phase layer
-// was the faster one with dense factors).
+// 73.40 vs 74.78).
 constexpr int64_t kDlContractMaxT = 4;
 constexpr int64_t kDlContractAutoPadded = 2;
 constexpr int64_t kDlContractAutoDense = 3;

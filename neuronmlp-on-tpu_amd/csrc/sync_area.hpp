@@ -1,7 +1,8 @@
 // The workspace's 4096-byte sync area: cross-block words of the kernels that
 // wait on other blocks (the persistent decode layers' grid barriers and
 // split-K tile counters, the large-tile GEMM's in-kernel split-K fixup), the
-// timeout flag and the bounded-wait override.  All words start at zero (the
+// arrival counters of the streaming stages' K splits (which nobody waits for),
+// the timeout flag and the bounded-wait override.  All words start at zero (the
 // caller zeroes the area once) and every launch leaves them valid for the next
 // one on the same workspace.
 #pragma once
@@ -32,8 +33,8 @@ constexpr int kDlSpin = kDlFlag + 1;
 constexpr int kGvDone = kDlFlag + kDlLine;
 constexpr uint64_t kGvDoneBad = (uint64_t)1 << 63;
 // 32-bit arrival counters of the split-K tiles of phases 1, 3 and 4 (in
-// that order) fill the rest of the 4 KB area, kDlTileLines 128-byte lines.
-// Tile t's counter is word t / kDlTileLines of line t % kDlTileLines, so
+// that order), and of a streaming stage's tiles, fill the rest of the 4 KB
+// area, kDlTileLines 128-byte lines.  Tile t's counter is word t / kDlTileLines of line t % kDlTileLines, so
 // neighbouring tiles, whose units finish together, hit different lines
 // (packed consecutively, ~100 blocks' atomics on 3 lines cost ~2 us per
 // layer).  The last arrival of a launch resets its tile's counter to zero.
