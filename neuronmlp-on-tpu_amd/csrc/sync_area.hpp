@@ -34,10 +34,11 @@ constexpr int kGvDone = kDlFlag + kDlLine;
 constexpr uint64_t kGvDoneBad = (uint64_t)1 << 63;
 // 32-bit arrival counters of the split-K tiles of phases 1, 3 and 4 (in
 // that order), and of a streaming stage's tiles, fill the rest of the 4 KB
-// area, kDlTileLines 128-byte lines.  Tile t's counter is word t / kDlTileLines of line t % kDlTileLines, so
-// neighbouring tiles, whose units finish together, hit different lines
-// (packed consecutively, ~100 blocks' atomics on 3 lines cost ~2 us per
-// layer).  The last arrival of a launch resets its tile's counter to zero.
+// area, kDlTileLines 128-byte lines.  Tile t's counter is word t /
+// kDlTileLines of line t % kDlTileLines, so neighbouring tiles, whose units
+// finish together, hit different lines (packed consecutively, ~100 blocks'
+// atomics on 3 lines cost ~2 us per layer).  The last arrival of a launch
+// resets its tile's counter to zero.
 constexpr int kDlTileWords = kGvDone + kDlLine;
 constexpr int kDlTileLines = (512 - kDlTileWords) / kDlLine;
 constexpr int kDlMaxTiles = kDlTileLines * 32;
